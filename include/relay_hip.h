@@ -350,8 +350,44 @@ int rh_w8_merge_rmsnorm(const float* workspace, int ksplit, int T, int H, const 
                         const float* norm_w, float eps, void* out, void* stream);
 int rh_w8_merge_rmsnorm_fits(int H);
 
+/* rh_qkv_post_to_cache on the raw K-range partials of the qkv product (rh_gemm_w8_partials
+ * with its scale, or rh_gemm_f16_partials with scale NULL; ksplit = 1 takes a plain [T, N]
+ * product): the merge, bias, RoPE, fp16 q and the cache rows in one launch. head_dim a
+ * multiple of 8; the workspace 16-byte aligned. No counterpart in relay. */
+int rh_qkv_post_merge(const float* workspace, int ksplit, const float* scale, int T, const float* bias,
+                      const float* inv_freq, const int* pos, const int* seq, const int* table_off, const int* tables,
+                      void* kpool, void* vpool, void* q_out, float q_scale, int heads, int kv_heads, int head_dim,
+                      int block_size, void* stream);
+
 /* The ksplit rh_gemm_w8_skinny uses for this shape (-1 outside its limits). */
 int rh_gemm_w8_split_plan(int T, int K, int N);
+
+/* y[t, n] = sum_k W16[n, k] * x[t, k] (+ beta * y[t, n] when beta != 0), any T >= 0: the fp16
+ * product above the skinny kernels' token range, fp32 sums in a fixed order. W16 [N, K] rows
+ * ldw elements apart (ldw >= K, a multiple of 8), x fp16 [T, K], y fp32 [T, N]; K a multiple
+ * of 64; W16, x and y 16-byte aligned; T * K and N * ldw below 2^30 (rh_gemm_f16_fits tests the
+ * shape). Replaces cublasGemmEx (cuda_backend.cu:726-730) at prefill and large decode batches. */
+int rh_gemm_f16(const void* w16, int64_t ldw, const void* x, float* y, int T, int K, int N, float beta, void* stream);
+int rh_gemm_f16_fits(int T, int K, int N);
+
+/* The raw sums of ksplit K ranges (2 <= ksplit <= 8, at most K / 64) of the same product into
+ * workspace [ksplit][T][N] (N a multiple of 4), for a consumer that adds them in order:
+ * rh_qkv_post_merge, rh_f16_merge_rmsnorm, rh_f16_merge_silu. rh_gemm_f16_partials_plan gives
+ * the split that is fastest with such a consumer (1: do not split). No counterpart in relay. */
+int rh_gemm_f16_partials(const void* w16, int64_t ldw, const void* x, int T, int K, int N, int ksplit,
+                         float* workspace, void* stream);
+int rh_gemm_f16_partials_plan(int T, int K, int N);
+int rh_f16_merge_silu(const float* workspace, int ksplit, int T, int I, void* act, void* stream);
+int rh_f16_merge_rmsnorm(const float* workspace, int ksplit, int T, int H, float* x, const float* norm_w, float eps,
+                         void* out, void* stream);
+
+/* act[t, a] = fp16(silu(g) * u) of the fused gate/up matrix W16 [2 I, K] (rows ldw elements
+ * apart) with x fp16 [T, K]: rh_gemm_f16 with SiLU * mul in its epilogue (act fp16 [T, I], 8-byte
+ * aligned). rh_gemm_f16_gate_up_plan gives 1 where this is the faster form, else the split
+ * for rh_gemm_f16_partials + rh_f16_merge_silu. No counterpart in relay (cublasGemmEx then
+ * silu_mul_kernel, cuda_backend.cu:588-589). */
+int rh_gemm_f16_gate_up_silu(const void* w16, int64_t ldw, const void* x, void* act, int T, int K, int I, void* stream);
+int rh_gemm_f16_gate_up_plan(int T, int K, int I);
 
 /* Per-row symmetric int8 quantization of an fp32 matrix [N, K] on the device:
  * scale[n] = max_k |w[n, k]| / 127 (1 if the row is all zero), q = round-half-even(w / scale),

@@ -82,6 +82,15 @@ SIGNATURES = {
     "rh_gemm_w8_kernel": (I, [I, I, I, I]),
     "rh_gemm_w8_gate_up_silu": (I, [P, I64, P, P, P, I, I, I, P]),
     "rh_gemm_w8_split_plan": (I, [I, I, I]),
+    "rh_qkv_post_merge": (I, [P, I, P, I, P, P, P, P, P, P, P, P, P, F, I, I, I, I, P]),
+    "rh_gemm_f16": (I, [P, I64, P, P, I, I, I, F, P]),
+    "rh_gemm_f16_fits": (I, [I, I, I]),
+    "rh_gemm_f16_partials": (I, [P, I64, P, I, I, I, I, P, P]),
+    "rh_gemm_f16_partials_plan": (I, [I, I, I]),
+    "rh_f16_merge_silu": (I, [P, I, I, I, P, P]),
+    "rh_f16_merge_rmsnorm": (I, [P, I, I, I, P, P, F, P, P]),
+    "rh_gemm_f16_gate_up_silu": (I, [P, I64, P, P, I, I, I, P]),
+    "rh_gemm_f16_gate_up_plan": (I, [I, I, I]),
     "rh_gemv_f16_rmsnorm": (I, [P, I64, P, P, F, P, I, I, I, F, P]),
     "rh_gemv_f16_silu": (I, [P, I64, P, P, I, I, I, F, P]),
     "rh_gemv_f16_fused_fits": (I, [I, I]),

@@ -1,6 +1,6 @@
 // relay's Backend on one MI355X: fp16 (or weight-only int8) weights and KV cache in HBM,
 // fp32 residual stream, the gfx950 kernels of include/relay_hip.h for attention and the
-// int8 GEMV, rocBLAS for the dense fp16 GEMMs.
+// int8 GEMV, the tile kernel (rh_gemm_f16) or hipBLASLt / rocBLAS for the dense fp16 GEMMs.
 //
 // The host orchestration mirrors CudaBackend (engine/src/cuda_backend.cu:311-759) in
 // contract, not in code:
@@ -214,6 +214,9 @@ class HipBackend final : public Backend {
   bool fused(const DeviceMatrix& W, int T, bool int8_ok = false) const;
   float* w8_split_ws(int ks, int T, int N);
   int w8_partials(const DeviceMatrix& W, const std::uint16_t* x, int T);
+  int partials(const DeviceMatrix& W, const std::uint16_t* x, int T);
+  // Whether an fp16 product runs the tile kernel (rh_gemm_f16) for this shape.
+  static bool tiled(int K, int N, int T);
   void gemm_f16(const std::uint16_t* W, const std::uint16_t* x, float* y, int T, int K, int N, float beta);
   // Whether gemm_f16 runs the skinny product (else the library GEMM) for this shape.
   static bool skinny(int K, int N, int T);
@@ -396,6 +399,10 @@ void HipBackend::gemm_f16(const std::uint16_t* W, const std::uint16_t* x, float*
     RH_CHECK(rh_gemv_f16_splitk(W, K, x, y, T, K, N, beta, ks, split_ws_.p, split_counters_.p, stream_));
     return;
   }
+  if (tiled(K, N, T) && W != dequant_.p) {
+    RH_CHECK(rh_gemm_f16(W, K, x, y, T, K, N, beta, stream_));
+    return;
+  }
   // Library products of the fp16 weights: hipBLASLt with a timed choice. A dequantized int8
   // copy (just written, read from the caches) stays on rocBLAS: measured faster there
   // (Llama-3 int8 mixed step 26.0 vs 26.7 ms).
@@ -413,6 +420,15 @@ bool HipBackend::skinny(int K, int N, int T) {
   // kernel: SmolLM2-135M 32 x 640 decode step 1.50 -> 1.27 ms; TinyLlama's 2048 x 2048 o
   // projection at 32 tokens 1.569 -> 1.592 ms against the library's).
   return K % 16 == 0 && (T <= 16 || (T <= 32 && static_cast<std::int64_t>(N) * K < (std::int64_t{1} << 22)));
+}
+
+bool HipBackend::tiled(int K, int N, int T) {
+  // The library's 256 x 256 kernels stay ahead on the largest products: library / tile kernel
+  // in isolation (us) 53 / 72 at 384 x 32000 outputs (K = 2048), 91 / 113 at 2048 x 6144
+  // (4096), 108 / 130 at 512 x 28672 (4096); 35 / 34 at 512 x 11264 (2048), 68 / 73 at 2048 x
+  // 4096 (4096), 93 / 72 at 512 x 4096 (14336), 58 / 53 at 2048 x 2048 (5632), 32 / 9.6 at
+  // 256 x 2048 (2048).
+  return !skinny(K, N, T) && rh_gemm_f16_fits(T, K, N) && static_cast<std::int64_t>(T) * N < 10000000;
 }
 
 bool HipBackend::fused(const DeviceMatrix& W, int T, bool int8_ok) const {
@@ -448,7 +464,18 @@ int HipBackend::w8_partials(const DeviceMatrix& W, const std::uint16_t* x, int T
   return ks;
 }
 
-// The K-range workspace of a split int8 product (grown on demand).
+// The same for either weight type: fp16 products on the tile kernel leave the ranges of its
+// plan (rh_f16_merge_* and rh_qkv_post_merge add them).
+int HipBackend::partials(const DeviceMatrix& W, const std::uint16_t* x, int T) {
+  if (W.i8.p) return w8_partials(W, x, T);
+  if (!tiled(W.K, W.N, T) || W.N % 4) return 0;
+  const int ks = rh_gemm_f16_partials_plan(T, W.K, W.N);
+  if (ks < 2) return 0;
+  RH_CHECK(rh_gemm_f16_partials(W.f16.p, W.K, x, T, W.K, W.N, ks, w8_split_ws(ks, T, W.N), stream_));
+  return ks;
+}
+
+// The K-range workspace of a split product (grown on demand).
 float* HipBackend::w8_split_ws(int ks, int T, int N) {
   if (ks <= 1) return nullptr;
   const std::size_t need = static_cast<std::size_t>(ks) * T * N;
@@ -612,6 +639,13 @@ std::size_t HipBackend::enqueue_forward(const ForwardBatch& batch, LayerObserver
   const float q_scale = scale * 1.4426950408889634f, attn_scale = 0.6931471805599453f;
   HIP_CHECK(hipEventRecord(fwd_begin_, stream_));
   RH_CHECK(rh_embed(d_tok, T, embed_.p, H, x_.p, stream_));
+  // x += the product whose ks partials are in split_ws_, xn = its RMSNorm.
+  auto merge_rmsnorm = [&](const DeviceMatrix& W, int ks, int rows, const float* norm) {
+    if (W.i8.p)
+      RH_CHECK(rh_w8_merge_rmsnorm(split_ws_.p, ks, rows, H, W.scale.p, x_.p, norm, eps, xn_.p, stream_));
+    else
+      RH_CHECK(rh_f16_merge_rmsnorm(split_ws_.p, ks, rows, H, x_.p, norm, eps, xn_.p, stream_));
+  };
   bool attn_xn_ready = false;  // the previous layer's fused down merge wrote this layer's xn
   for (int l = 0; l < c_.layers; ++l) {
     DeviceLayer& L = layers_[l];
@@ -643,16 +677,21 @@ std::size_t HipBackend::enqueue_forward(const ForwardBatch& batch, LayerObserver
                (T <= 16 || (T <= rh_gemv_f16_max_tokens() && QKV <= 4096)) && rh_gemv_f16_split_plan(T, H, QKV) == 1) {
       // (17-32 tokens: TinyLlama's 2560-row qkv 11.1 us on the 16-row tile against 9.5 + 3.0 us
       // for the library product and a separate qkv_post; the whole-line kernel since: 32 x 2048
-      // decode step 1.638 -> 1.573-1.603 ms.)
+      // decode step 1.638 -> 1.573-1.603 ms; at 32 tokens 9.1 us in the step against 6.0 + 5.1
+      // for the tile kernel's ranges and rh_qkv_post_merge.)
       // The projection and qkv_post in one launch (the RMSNorm cannot be folded in here).
       if (!attn_xn_ready) RH_CHECK(rh_rmsnorm(x_.p, nullptr, T, L.attn_norm.p, H, eps, xn_.p, stream_));
       RH_CHECK(rh_gemv_f16_qkv(L.wqkv.f16.p, H, xn_.p, qkv_.p, T, H, bias, inv_freq_.p, d_pos, d_seq, d_toff, d_tab,
                                kc, vc, q_out, q_scale, c_.heads, c_.kv_heads, D, layout_.block_size, stream_));
     } else {
       if (!attn_xn_ready) RH_CHECK(rh_rmsnorm(x_.p, nullptr, T, L.attn_norm.p, H, eps, xn_.p, stream_));
-      gemm(L.wqkv, xn_.p, qkv_.p, T, 0.0f);
+      const int ks = q_out && D % 8 == 0 ? partials(L.wqkv, xn_.p, T) : 0;
+      if (!ks) gemm(L.wqkv, xn_.p, qkv_.p, T, 0.0f);
       // The fast kernels read only the fp16 q and the cache; the reference kernel reads qkv.
-      if (q_out)
+      if (ks)
+        RH_CHECK(rh_qkv_post_merge(split_ws_.p, ks, L.wqkv.scale.p, T, bias, inv_freq_.p, d_pos, d_seq, d_toff, d_tab, kc,
+                                   vc, q_out, q_scale, c_.heads, c_.kv_heads, D, layout_.block_size, stream_));
+      else if (q_out)
         RH_CHECK(rh_qkv_post_to_cache(qkv_.p, T, bias, inv_freq_.p, d_pos, d_seq, d_toff, d_tab, kc, vc, q_out,
                                       q_scale, c_.heads, c_.kv_heads, D, layout_.block_size, stream_));
       else
@@ -680,8 +719,8 @@ std::size_t HipBackend::enqueue_forward(const ForwardBatch& batch, LayerObserver
     // launches fewer per layer).
     bool mlp_xn_ready = false;
     const bool merge_norm = rh_w8_merge_rmsnorm_fits(H);
-    if (const int ks = merge_norm ? w8_partials(L.wo, attn_.p, T) : 0) {
-      RH_CHECK(rh_w8_merge_rmsnorm(split_ws_.p, ks, T, H, L.wo.scale.p, x_.p, L.mlp_norm.p, eps, xn_.p, stream_));
+    if (const int ks = merge_norm ? partials(L.wo, attn_.p, T) : 0) {
+      merge_rmsnorm(L.wo, ks, T, L.mlp_norm.p);
       mlp_xn_ready = true;
     } else {
       gemm(L.wo, attn_.p, x_.p, T, 1.0f);  // x += attn W_o^T
@@ -711,8 +750,23 @@ std::size_t HipBackend::enqueue_forward(const ForwardBatch& batch, LayerObserver
         const bool tile_silu = L.w_gate_up.i8.p && T > 64 && rh_gemm_w8_plan(T, H, 2 * I) == 1 &&
                                rh_gemm_w8_kernel(T, H, 2 * I, 1) == 1 &&
                                (static_cast<std::int64_t>(I) + 256) * L.w_gate_up.ldw < (std::int64_t(1) << 31);
-        const int ks = tile_silu || I % 8 ? 0 : w8_partials(L.w_gate_up, xn_.p, T);
-        if (tile_silu) {
+        // fp16 above the whole-line kernel's range: SiLU·mul in the tile kernel's epilogue. On
+        // products large enough for the library that saves the fp32 [T, 2 I] round trip and
+        // a launch, which outweighs the library's faster kernel while K is short (2048 tokens
+        // of TinyLlama: 104 us against 97 + 22; 512 of Llama-3-8B: 130 against 106 + 12).
+        const bool f16_tile = !L.w_gate_up.i8.p && !skinny(H, 2 * I, T) &&
+                              (tiled(H, 2 * I, T) || (H <= 2048 && rh_gemm_f16_fits(T, H, 2 * I)));
+        const int ks = tile_silu || f16_tile || I % 8 ? 0 : w8_partials(L.w_gate_up, xn_.p, T);
+        if (f16_tile) {
+          const int gks = rh_gemm_f16_gate_up_plan(T, H, I);
+          if (gks > 1) {
+            RH_CHECK(rh_gemm_f16_partials(L.w_gate_up.f16.p, H, xn_.p, T, H, 2 * I, gks, w8_split_ws(gks, T, 2 * I), stream_));
+            RH_CHECK(rh_f16_merge_silu(split_ws_.p, gks, T, I, act_.p, stream_));
+          } else {
+            RH_CHECK(rh_gemm_f16_gate_up_silu(L.w_gate_up.f16.p, H, xn_.p, act_.p, T, H, I, stream_));
+          }
+          act_ready = true;
+        } else if (tile_silu) {
           RH_CHECK(rh_gemm_w8_gate_up_silu(L.w_gate_up.i8.p, L.w_gate_up.ldw, L.w_gate_up.scale.p, xn_.p, act_.p, T, H,
                                            I, stream_));
           act_ready = true;
@@ -741,10 +795,9 @@ std::size_t HipBackend::enqueue_forward(const ForwardBatch& batch, LayerObserver
       RH_CHECK(rh_gemv_f16_silu(L.w_down.f16.p, I, gu_.p, x_.p, T, I, H, 1.0f, stream_));  // x += act W_down^T
     } else {
       if (!act_ready) RH_CHECK(rh_silu_mul(gu_.p, T, I, act_.p, stream_));
-      const int ks = merge_norm && l + 1 < c_.layers ? w8_partials(L.w_down, act_.p, T) : 0;
-      if (ks) {  // x += act W_down^T, then the next layer's attention RMSNorm
-        RH_CHECK(rh_w8_merge_rmsnorm(split_ws_.p, ks, T, H, L.w_down.scale.p, x_.p, layers_[l + 1].attn_norm.p, eps,
-                                     xn_.p, stream_));
+      const int ks = merge_norm ? partials(L.w_down, act_.p, T) : 0;
+      if (ks) {  // x += act W_down^T, then the next layer's attention RMSNorm (or the final one)
+        merge_rmsnorm(L.w_down, ks, T, l + 1 < c_.layers ? layers_[l + 1].attn_norm.p : final_norm_.p);
         attn_xn_ready = true;
       } else {
         gemm(L.w_down, act_.p, x_.p, T, 1.0f);  // x += act W_down^T
@@ -752,7 +805,8 @@ std::size_t HipBackend::enqueue_forward(const ForwardBatch& batch, LayerObserver
     }
   }
   if (R) {
-    RH_CHECK(rh_rmsnorm(x_.p, d_rows, R, final_norm_.p, H, eps, xn_.p, stream_));
+    // The last merge wrote the final norm of every row: of the wanted ones when all are.
+    if (!(attn_xn_ready && R == T)) RH_CHECK(rh_rmsnorm(x_.p, d_rows, R, final_norm_.p, H, eps, xn_.p, stream_));
     gemm_f16(lm_head_.n ? lm_head_.p : embed_.p, xn_.p, logits_.p, R, H, V, 0.0f);
   }
   HIP_CHECK(hipEventRecord(fwd_end_, stream_));

@@ -133,9 +133,10 @@ __global__ void rmsnorm_vec_kernel(const float* x, const int* rows, const float*
   }
 }
 
-// ---- the K-range merge of a split int8 product, fused into its consumer ----------------
+// ---- the K-range merge of a split product, fused into its consumer ----------------------
 //
-// rh_gemm_w8_partials leaves ksn raw partial planes ws[z][t][n]. The merge of a split product
+// rh_gemm_w8_partials and rh_gemm_f16_partials leave ksn raw partial planes ws[z][t][n] (fp16
+// weights have no scale: sc is null and the sum is the value). The merge of a split product
 // (w8_split_merge_kernel) computes y = (sum_z ws[z]) * scale (+ beta y, the ranges added in
 // order); these kernels do that merge for the product's consumer in the same launch, with
 // the same arithmetic, so that a decode step saves the merge launch (~4.5 us at T = 32).
@@ -153,6 +154,7 @@ __device__ __forceinline__ float4 merged4(const float* ws, int ksn, int64_t plan
 #pragma unroll
   for (int z = 0; z < kMaxMergeSplit; ++z)
     if (z < ksn) v = float4{v.x + p[z].x, v.y + p[z].y, v.z + p[z].z, v.w + p[z].w};
+  if (!sc) return v;
   return float4{mul_rounded(v.x, sc[0]), mul_rounded(v.y, sc[1]), mul_rounded(v.z, sc[2]), mul_rounded(v.w, sc[3])};
 }
 
@@ -163,9 +165,10 @@ __global__ void w8_merge_silu_kernel(const float* __restrict__ ws, int ksn, int 
   const int t = blockIdx.x, i = (blockIdx.y * kThreads + threadIdx.x) * 8;
   if (i >= I) return;
   const int64_t plane = static_cast<int64_t>(T) * 2 * I, row = static_cast<int64_t>(t) * 2 * I;
-  const float4 g0 = merged4(ws, ksn, plane, row + i, scale + i), g1 = merged4(ws, ksn, plane, row + i + 4, scale + i + 4);
-  const float4 u0 = merged4(ws, ksn, plane, row + I + i, scale + I + i),
-               u1 = merged4(ws, ksn, plane, row + I + i + 4, scale + I + i + 4);
+  const float *sg = scale ? scale + i : nullptr, *su = scale ? scale + I + i : nullptr;
+  const float4 g0 = merged4(ws, ksn, plane, row + i, sg), g1 = merged4(ws, ksn, plane, row + i + 4, sg ? sg + 4 : sg);
+  const float4 u0 = merged4(ws, ksn, plane, row + I + i, su),
+               u1 = merged4(ws, ksn, plane, row + I + i + 4, su ? su + 4 : su);
   const float gv[8] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w};
   const float uv[8] = {u0.x, u0.y, u0.z, u0.w, u1.x, u1.y, u1.z, u1.w};
   half8 r;
@@ -194,7 +197,7 @@ __global__ void w8_merge_rmsnorm_kernel(const float* __restrict__ ws, int ksn, i
     const int j = threadIdx.x + i * kThreads;
     if (j < n4) {
       const float4 old = xr[j];
-      const float4 m = merged4(ws, ksn, plane, row + 4 * j, scale + 4 * j);
+      const float4 m = merged4(ws, ksn, plane, row + 4 * j, scale ? scale + 4 * j : nullptr);
       xv[i] = float4{m.x + old.x, m.y + old.y, m.z + old.z, m.w + old.w};
       xr[j] = xv[i];
       wv[i] = wr[j];
@@ -266,6 +269,55 @@ __global__ void qkv_post_kernel(float* qkv, const float* bias, const float* inv_
   half_t* dst = (h < heads + kv_heads ? kc : vc) + kv_row_offset(block, kv_heads, kvh, block_size, slot, D);
   dst[i] = static_cast<half_t>(a);
   dst[i + half] = static_cast<half_t>(b);
+}
+
+// qkv_post_kernel<false> on the ksn partial planes of the qkv product (merged4, then the same
+// arithmetic per element); a thread takes four consecutive pairs, D a multiple of 8. Bound by
+// latency and the planes' reads: 512 tokens of TinyLlama (2 planes, 10.5 MB) 4.9 us, where the
+// one-plane kernel's scalar loads take 4.3 us on half the bytes.
+__global__ void qkv_post_merge_kernel(const float* __restrict__ ws, int ksn, const float* __restrict__ scale, int T,
+                                      const float* bias, const float* inv_freq, const int* pos, const int* seq,
+                                      const int* table_off, const int* tables, half_t* kc, half_t* vc, half_t* q_out,
+                                      float q_scale, int heads, int kv_heads, int D, int block_size) {
+  const int t = blockIdx.x, half = D / 2, quads = half / 4;
+  const int idx = blockIdx.y * kThreads + threadIdx.x;
+  if (idx >= (heads + 2 * kv_heads) * quads) return;
+  const int Q = heads * D, QKV = Q + 2 * kv_heads * D;
+  const int h = idx / quads, i = 4 * (idx % quads), n = h * D + i;
+  const int64_t plane = static_cast<int64_t>(T) * QKV, row = static_cast<int64_t>(t) * QKV;
+  const float4 va = merged4(ws, ksn, plane, row + n, scale ? scale + n : nullptr);
+  const float4 vb = merged4(ws, ksn, plane, row + n + half, scale ? scale + n + half : nullptr);
+  const int p = pos[t];
+  half_t* dst;
+  if (h < heads) {
+    dst = q_out + static_cast<int64_t>(t) * Q + n;
+  } else {
+    const int block = tables[table_off[seq[t]] + p / block_size], slot = p % block_size;
+    dst = (h < heads + kv_heads ? kc : vc) + kv_row_offset(block, kv_heads, (h - heads) % kv_heads, block_size, slot, D) + i;
+  }
+  float a[4] = {va.x, va.y, va.z, va.w}, b[4] = {vb.x, vb.y, vb.z, vb.w};
+  half4 oa, ob;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    if (bias) {
+      a[e] += bias[n + e];
+      b[e] += bias[n + e + half];
+    }
+    if (h < heads + kv_heads) {
+      const float angle = static_cast<float>(p) * inv_freq[i + e];
+      float sn, cs;
+      sincosf(angle, &sn, &cs);
+      // Products rounded before the add (no fused multiply-add), as the CPU computes them.
+      const float ra = __fsub_rn(__fmul_rn(a[e], cs), __fmul_rn(b[e], sn));
+      const float rb = __fadd_rn(__fmul_rn(b[e], cs), __fmul_rn(a[e], sn));
+      a[e] = ra;
+      b[e] = rb;
+    }
+    oa[e] = h < heads ? f16_of_product(a[e], q_scale) : static_cast<half_t>(a[e]);
+    ob[e] = h < heads ? f16_of_product(b[e], q_scale) : static_cast<half_t>(b[e]);
+  }
+  *reinterpret_cast<half4*>(dst) = oa;
+  *reinterpret_cast<half4*>(dst + half) = ob;
 }
 
 __global__ void silu_mul_kernel(const float* gu, int I, half_t* act) {
@@ -530,30 +582,73 @@ int rh_silu_mul(const float* gu, int T, int I, void* act, void* stream) {
   return 0;
 }
 
-int rh_w8_merge_silu(const float* workspace, int ksplit, int T, int I, const float* scale, void* act, void* stream) {
-  if (T == 0) return 0;
+static int merge_silu(const float* workspace, int ksplit, int T, int I, const float* scale, void* act, void* stream) {
   RH_REQUIRE(T > 0 && I > 0 && I % 8 == 0 && ksplit >= 1 && ksplit <= kMaxMergeSplit,
-             "w8_merge_silu: I must be a positive multiple of 8 and ksplit in 1..8");
-  RH_REQUIRE(workspace && scale && act && reinterpret_cast<uintptr_t>(act) % 16 == 0, "w8_merge_silu: bad pointer");
+             "merge_silu: I must be a positive multiple of 8 and ksplit in 1..8");
+  RH_REQUIRE(workspace && act && reinterpret_cast<uintptr_t>(act) % 16 == 0, "merge_silu: bad pointer");
   RH_TRY_LAUNCH(hipLaunchKernelGGL(w8_merge_silu_kernel, dim3(T, (I + 8 * kThreads - 1) / (8 * kThreads)),
                                    dim3(kThreads), 0, static_cast<hipStream_t>(stream), workspace, ksplit, T, I, scale,
                                    static_cast<half_t*>(act)));
   return 0;
 }
 
+int rh_w8_merge_silu(const float* workspace, int ksplit, int T, int I, const float* scale, void* act, void* stream) {
+  if (T == 0) return 0;
+  RH_REQUIRE(scale != nullptr, "w8_merge_silu: bad pointer");
+  return merge_silu(workspace, ksplit, T, I, scale, act, stream);
+}
+
+int rh_f16_merge_silu(const float* workspace, int ksplit, int T, int I, void* act, void* stream) {
+  if (T == 0) return 0;
+  return merge_silu(workspace, ksplit, T, I, nullptr, act, stream);
+}
+
 int rh_w8_merge_rmsnorm_fits(int H) { return H > 0 && H % 4 == 0 && H <= 4 * kRmsVec * kThreads; }
+
+static int merge_rmsnorm(const float* workspace, int ksplit, int T, int H, const float* scale, float* x,
+                         const float* norm_w, float eps, void* out, void* stream) {
+  RH_REQUIRE(T > 0 && rh_w8_merge_rmsnorm_fits(H) && ksplit >= 1 && ksplit <= kMaxMergeSplit,
+             "merge_rmsnorm: H must be a multiple of 4, at most 4096, and ksplit in 1..8");
+  RH_REQUIRE(workspace && x && norm_w && out &&
+                 (reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(norm_w) |
+                  reinterpret_cast<uintptr_t>(out)) % 16 == 0,
+             "merge_rmsnorm: x, norm_w and out must be 16-byte aligned");
+  RH_TRY_LAUNCH(hipLaunchKernelGGL(w8_merge_rmsnorm_kernel, dim3(T), dim3(kThreads), 0, static_cast<hipStream_t>(stream),
+                                   workspace, ksplit, T, H, scale, x, norm_w, eps, static_cast<half_t*>(out)));
+  return 0;
+}
 
 int rh_w8_merge_rmsnorm(const float* workspace, int ksplit, int T, int H, const float* scale, float* x,
                         const float* norm_w, float eps, void* out, void* stream) {
   if (T == 0) return 0;
-  RH_REQUIRE(T > 0 && rh_w8_merge_rmsnorm_fits(H) && ksplit >= 1 && ksplit <= kMaxMergeSplit,
-             "w8_merge_rmsnorm: H must be a multiple of 4, at most 4096, and ksplit in 1..8");
-  RH_REQUIRE(workspace && scale && x && norm_w && out &&
-                 (reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(norm_w) |
-                  reinterpret_cast<uintptr_t>(out)) % 16 == 0,
-             "w8_merge_rmsnorm: x, norm_w and out must be 16-byte aligned");
-  RH_TRY_LAUNCH(hipLaunchKernelGGL(w8_merge_rmsnorm_kernel, dim3(T), dim3(kThreads), 0, static_cast<hipStream_t>(stream),
-                                   workspace, ksplit, T, H, scale, x, norm_w, eps, static_cast<half_t*>(out)));
+  RH_REQUIRE(scale != nullptr, "w8_merge_rmsnorm: scale is required");
+  return merge_rmsnorm(workspace, ksplit, T, H, scale, x, norm_w, eps, out, stream);
+}
+
+int rh_f16_merge_rmsnorm(const float* workspace, int ksplit, int T, int H, float* x, const float* norm_w, float eps,
+                         void* out, void* stream) {
+  if (T == 0) return 0;
+  return merge_rmsnorm(workspace, ksplit, T, H, nullptr, x, norm_w, eps, out, stream);
+}
+
+int rh_qkv_post_merge(const float* workspace, int ksplit, const float* scale, int T, const float* bias,
+                      const float* inv_freq, const int* pos, const int* seq, const int* table_off, const int* tables,
+                      void* kpool, void* vpool, void* q_out, float q_scale, int heads, int kv_heads, int head_dim,
+                      int block_size, void* stream) {
+  if (T == 0) return 0;
+  RH_REQUIRE(T > 0 && heads > 0 && kv_heads > 0 && head_dim > 0 && head_dim % 8 == 0 && block_size > 0,
+             "qkv_post_merge: head_dim must be a positive multiple of 8");
+  RH_REQUIRE(workspace && q_out && kpool && vpool && ksplit >= 1 && ksplit <= kMaxMergeSplit,
+             "qkv_post_merge: missing pointer, or ksplit not in 1..8");
+  RH_REQUIRE(reinterpret_cast<uintptr_t>(workspace) % 16 == 0 &&
+                 (reinterpret_cast<uintptr_t>(q_out) | reinterpret_cast<uintptr_t>(kpool) |
+                  reinterpret_cast<uintptr_t>(vpool)) % 8 == 0,
+             "qkv_post_merge: the workspace must be 16-byte aligned, q_out and the pools 8-byte");
+  const int quads = (heads + 2 * kv_heads) * (head_dim / 8);
+  RH_TRY_LAUNCH(hipLaunchKernelGGL(qkv_post_merge_kernel, dim3(T, (quads + kThreads - 1) / kThreads), dim3(kThreads), 0,
+                                   static_cast<hipStream_t>(stream), workspace, ksplit, scale, T, bias, inv_freq, pos,
+                                   seq, table_off, tables, static_cast<half_t*>(kpool), static_cast<half_t*>(vpool),
+                                   static_cast<half_t*>(q_out), q_scale, heads, kv_heads, head_dim, block_size));
   return 0;
 }
 
