@@ -5,14 +5,16 @@
 // (a chunk at an offset sees the earlier chunks' keys). Re-cut for 64-wide waves and 32x32
 // matrix cores:
 //
-// - Work unit: one workgroup of eight waves per (work item, query head). A work item is a
+// - Work unit: one workgroup of eight waves per (work item, query head), or per 64 or 32 rows
+//   of it where that leaves CUs idle (launch). A work item is a
 //   block of up to 128 consecutive rows of one chunk, or a pair of blocks (i, n-1-i) of
 //   the same chunk processed one after the other, so that every workgroup does the same
 //   causal work (rh_prefill_plan makes the items; it pairs when the grid is large).
-// - Waves r and r+4 (the two waves of one SIMD) own the block's rows 32r .. 32r+31 and
-//   split every key tile (128 keys at head_dim 64, 64 at 128): the first half goes to wave
-//   r, the second to wave r+4. Each keeps its own running offset, sum and O^T; at the end of
-//   the block wave r+4 hands them to wave r through LDS. So two waves stay busy on every SIMD
+// - With 128 rows, waves r and r+4 (the two waves of one SIMD) own the block's rows 32r ..
+//   32r+31 and split every key tile (128 keys at head_dim 64, 64 at 128): the first half goes
+//   to wave r, the second to wave r+4 (with 64 or 32 rows four or eight waves share a strip
+//   and a tile has a part of 32 keys for each). Each keeps its own running offset, sum and
+//   O^T; at the end of the block the later parts' waves hand them to the first's through LDS. So two waves stay busy on every SIMD
 //   until the block's last tile (with one wave per 32-row strip, every SIMD drops to one wave
 //   once the short blocks finish), and each SIMD holds one wave of each half (the second
 //   halves carry more of the diagonal's work).
@@ -49,14 +51,14 @@
 namespace relay_hip {
 namespace {
 
-constexpr int kRows = 128;    // query rows per block
-constexpr int kWaves = 8;     // two per 32-row strip
+constexpr int kRows = 128;    // query rows per block of a work item
+constexpr int kWaves = 8;     // SPLIT per 32-row strip
 constexpr int kThreads = kWaves * kWave;
 // 32-key sub-steps per wave per tile: at D 64 two independent S^T chains per wave under
 // one softmax (measured 45.0 -> 41.8 us at config 3); at D 128 the second chain's
 // registers would spill.
-template <int D>
-constexpr int sub_steps() { return D == 128 ? 1 : 2; }
+template <int D, int SPLIT>
+constexpr int sub_steps() { return D == 128 || SPLIT > 2 ? 1 : 2; }
 
 // One work item: block a (t0, rows, first position), block b likewise (rows 0: none), and
 // the chunk's block-table offset. Layout of rh_prefill_plan's int32[8] records.
@@ -102,11 +104,16 @@ __device__ __forceinline__ int kswz(int key) {
 
 // D is the compute width, DR the head size of the cache rows, q and out: equal, except head
 // size 16, which runs at width 32 with dims 16..31 of K, V and q taken as zero.
-template <int D, int DR, bool POW2>
+// SPLIT: how many waves share a 32-row strip, i.e. key parts per tile (2, 4 or 8); a workgroup
+// then takes 32 * 8 / SPLIT rows, kSubs workgroups a block.
+template <int D, int DR, bool POW2, int SPLIT>
 __global__ __launch_bounds__(kThreads) void flash_prefill_kernel(const PrefillArgs a) {
   static_assert(DR == D || (DR == 16 && D == 32), "head size 16 runs at width 32");
-  constexpr int kSub = sub_steps<D>();      // 32-key sub-steps per wave per tile
-  constexpr int kKeyTile = 64 * kSub;       // keys per LDS tile
+  constexpr int kSub = sub_steps<D, SPLIT>();   // 32-key sub-steps per wave per tile
+  constexpr int kKeyTile = 32 * SPLIT * kSub;   // keys per LDS tile
+  constexpr int kStrips = kWaves / SPLIT;       // 32-row strips per workgroup
+  constexpr int kWgRows = 32 * kStrips;
+  constexpr int kSubs = kRows / kWgRows;        // workgroups per block of rows
   constexpr int CH = D / 8;                                 // 16-byte chunks per row
   constexpr int MK = D / 16;                                // QK MFMAs per half tile
   constexpr int DT = D / 32;                                // 32-dim tiles of O^T
@@ -115,7 +122,7 @@ __global__ __launch_bounds__(kThreads) void flash_prefill_kernel(const PrefillAr
   constexpr int LOADS = 2 * PAIRS;                          // rows per thread per tile, each of K and V
   constexpr int KBUF = kKeyTile * D, VBUF = D * kKeyTile;   // halves per buffer
   constexpr int XSTRIP = DT * 16 * 64 + 2 * 64;             // floats per strip for the merge
-  constexpr int SMEM = std::max(2 * KBUF + 2 * VBUF, 2 * 4 * XSTRIP);
+  constexpr int SMEM = std::max(2 * KBUF + 2 * VBUF, 2 * kStrips * (SPLIT - 1) * XSTRIP);
 
   // Two K and two V buffers (row-major, 16-byte chunks XOR-swizzled by key); reused for the
   // merge of the half-tile partials.
@@ -125,7 +132,7 @@ __global__ __launch_bounds__(kThreads) void flash_prefill_kernel(const PrefillAr
 
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int c = lane & 31, hh = lane >> 5;
-  const int strip = w & 3, half = w >> 2;
+  const int strip = w % kStrips, half = w / kStrips;  // half: this wave's part of every tile
 
   // Workgroup -> (work item, head).
   const int b = blockIdx.x;
@@ -138,6 +145,9 @@ __global__ __launch_bounds__(kThreads) void flash_prefill_kernel(const PrefillAr
     wi = b / a.heads;
     head = b % a.heads;
   }
+  // The later rows of a block (more keys) first.
+  const int sub = kSubs - 1 - wi % kSubs;
+  wi /= kSubs;
   if (wi >= a.n_work) return;
   const PrefillWork wk = a.work[wi];
   const int kvh = head / (a.heads / a.kv_heads);
@@ -159,8 +169,10 @@ __global__ __launch_bounds__(kThreads) void flash_prefill_kernel(const PrefillAr
   };
 
   for (int phase = 0; phase < 2; ++phase) {
-    const int t0 = phase ? wk.t0b : wk.t0a, nrows = phase ? wk.nb : wk.na, p0 = phase ? wk.p0b : wk.p0a;
-    if (nrows <= 0) break;
+    const int r0 = sub * kWgRows;  // this workgroup's first row of the block
+    const int t0 = (phase ? wk.t0b : wk.t0a) + r0, p0 = (phase ? wk.p0b : wk.p0a) + r0;
+    const int nrows = min(kWgRows, (phase ? wk.nb : wk.na) - r0);
+    if (nrows <= 0) continue;
     const int nkeys = p0 + nrows;
     const int row = strip * 32 + c;
     const bool row_ok = row < nrows;
@@ -376,26 +388,32 @@ __global__ __launch_bounds__(kThreads) void flash_prefill_kernel(const PrefillAr
       __syncthreads();
     }
 
-    // Merge the strip's two halves: the odd wave's (max, sum, O^T) through LDS (the tile
-    // buffers are free after the loop's last barrier).
-    float* const xo = reinterpret_cast<float*>(smem) + strip * XSTRIP;
-    float* const xml = xo + DT * 16 * 64;
+    // Merge the strip's parts: the others' (max, sum, O^T) through LDS (the tile buffers are
+    // free after the loop's last barrier) into the first part's wave, which saw key 0, so its
+    // offset is finite; the others' may not be.
+    float* const xs = reinterpret_cast<float*>(smem) + strip * (SPLIT - 1) * XSTRIP;
     if (half) {
+      float* const xo = xs + (half - 1) * XSTRIP;
 #pragma unroll
       for (int i = 0; i < DT; ++i)
 #pragma unroll
         for (int r = 0; r < 16; ++r) xo[(i * 16 + r) * 64 + lane] = o[i][r];
-      xml[lane] = ref;
-      xml[64 + lane] = l_part;
+      xo[DT * 16 * 64 + lane] = ref;
+      xo[DT * 16 * 64 + 64 + lane] = l_part;
     }
     __syncthreads();
     if (!half && row_ok) {
-      // The even wave saw key 0, so its offset is finite; the odd one's may not be.
-      const float m_b = xml[lane], l_b = xml[64 + lane];
-      const float m = fmaxf(ref, m_b);
-      const float fa = fast_exp2(ref - m);
-      const float fb = m_b == -INFINITY ? 0.0f : fast_exp2(m_b - m);
-      const float l = l_part * fa + l_b * fb;
+      float f[SPLIT], m = ref;
+#pragma unroll
+      for (int p = 1; p < SPLIT; ++p) m = fmaxf(m, xs[(p - 1) * XSTRIP + DT * 16 * 64 + lane]);
+      f[0] = fast_exp2(ref - m);
+      float l = l_part * f[0];
+#pragma unroll
+      for (int p = 1; p < SPLIT; ++p) {
+        const float* const xml = xs + (p - 1) * XSTRIP + DT * 16 * 64;
+        f[p] = xml[lane] == -INFINITY ? 0.0f : fast_exp2(xml[lane] - m);
+        l += xml[64 + lane] * f[p];
+      }
       const float inv = 1.0f / (l + xlane_sum(l));
       half_t* orow = a.out + static_cast<int64_t>(t0 + row) * a.out_stride + static_cast<int64_t>(head) * DR;
 #pragma unroll
@@ -406,7 +424,10 @@ __global__ __launch_bounds__(kThreads) void flash_prefill_kernel(const PrefillAr
 #pragma unroll
           for (int j = 0; j < 4; ++j) {
             const int r = 4 * r4 + j;
-            v[j] = static_cast<half_t>((o[dt][r] * fa + xo[(dt * 16 + r) * 64 + lane] * fb) * inv);
+            float ov = o[dt][r] * f[0];
+#pragma unroll
+            for (int p = 1; p < SPLIT; ++p) ov += xs[(p - 1) * XSTRIP + (dt * 16 + r) * 64 + lane] * f[p];
+            v[j] = static_cast<half_t>(ov * inv);
           }
           if (DR == D || 32 * dt + 8 * r4 + 4 * hh < DR) *reinterpret_cast<half4*>(orow + 32 * dt + 8 * r4 + 4 * hh) = v;
         }
@@ -414,15 +435,31 @@ __global__ __launch_bounds__(kThreads) void flash_prefill_kernel(const PrefillAr
   }
 }
 
-template <int D, int DR>
-int launch(const PrefillArgs& a, hipStream_t s) {
-  const int grid = a.n_work * a.heads;
+template <int D, int DR, int SPLIT>
+int launch_split(const PrefillArgs& a, hipStream_t s) {
+  const int grid = a.n_work * a.heads * (SPLIT / 2);
   if (a.bs_shift >= 0) {
-    RH_TRY_LAUNCH(hipLaunchKernelGGL((flash_prefill_kernel<D, DR, true>), dim3(grid), dim3(kThreads), 0, s, a));
+    RH_TRY_LAUNCH(hipLaunchKernelGGL((flash_prefill_kernel<D, DR, true, SPLIT>), dim3(grid), dim3(kThreads), 0, s, a));
   } else {
-    RH_TRY_LAUNCH(hipLaunchKernelGGL((flash_prefill_kernel<D, DR, false>), dim3(grid), dim3(kThreads), 0, s, a));
+    RH_TRY_LAUNCH(hipLaunchKernelGGL((flash_prefill_kernel<D, DR, false, SPLIT>), dim3(grid), dim3(kThreads), 0, s, a));
   }
   return 0;
+}
+
+template <int D, int DR>
+int launch(const PrefillArgs& a, hipStream_t s) {
+  // Blocks of 128 rows that would leave CUs idle are cut into 64- or 32-row workgroups, whose
+  // waves share more of each tile's keys: up to one workgroup per CU. Measured (us, 128 / 64 /
+  // 32 rows; 32 q heads unless stated): D128, 8 kv heads, 512 rows at position 7680 147.7 /
+  // 104.4, 512 at 0 15.9 / 12.6, 100 at 4000 77.1 / 52.5; D64, 4 kv heads, 512 at 1536 25.2 /
+  // 19.9 / 27.5, 100 at 1000 16.1 / 12.3 / 11.1, 9 heads, 500 at 1500 24.7 / 18.7 / 15.1.
+  // Past the line a second round costs more than the finer deal gives: D128, 768 at 2000 (192
+  // blocks) 55.6 / 64.6, D64, 768 at 1000 23.3 / 26.0 / 35.3. At head size 128 the 32-row form's
+  // tiles (two buffers of 256 keys) do not fit the LDS.
+  const int64_t blocks = static_cast<int64_t>(a.n_work) * a.heads;
+  if constexpr (D <= 64)
+    if (blocks <= 64) return launch_split<D, DR, 8>(a, s);
+  return blocks <= 128 ? launch_split<D, DR, 4>(a, s) : launch_split<D, DR, 2>(a, s);
 }
 
 }  // namespace

@@ -127,6 +127,17 @@ def test_paired_blocks(torch_mod, dev, D):
     check_close(run_prefill(torch_mod, dev, case), oracle_out(case))
 
 
+@pytest.mark.parametrize("rows,start", [(1, 40), (33, 0), (65, 300), (97, 31), (128, 130), (225, 0)])
+@pytest.mark.parametrize("heads,kv_heads,D,bs", [(64, 8, 64, 16), (65, 5, 64, 12), (64, 4, 32, 16), (33, 3, 16, 16),
+                                                 (128, 8, 128, 16), (129, 3, 128, 16), (64, 8, 128, 5)])
+def test_row_cuts(torch_mod, dev, heads, kv_heads, D, bs, rows, start):
+    """Workgroups of 32, 64 and 128 rows, chosen by the number of (128-row block, head) pairs:
+    64 and 128 pairs are the largest of the first two, and a second block doubles the count.
+    Rows end before, at and past each workgroup's; early key parts of a row may be all masked."""
+    case = PagedCase([start + rows], [rows], heads, kv_heads, D, bs, seed=rows + heads)
+    check_close(run_prefill(torch_mod, dev, case), oracle_out(case))
+
+
 def test_gather_is_bit_exact_under_permutation(torch_mod, dev):
     case = PagedCase([400], [400], 8, 2, 64, 16, seed=1)
     a = run_prefill(torch_mod, dev, case)
