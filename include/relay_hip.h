@@ -412,6 +412,12 @@ int rh_embed(const int* tokens, int T, const void* table, int H, float* x, void*
  * (cuda_backend.cu:157-167) */
 int rh_rmsnorm(const float* x, const int* rows, int R, const float* w, int H, float eps, void* out, void* stream);
 
+/* x_out[r] = x[rows[r]] (fp32 [., H]) and a_out[r] = a[rows[r]] (fp16 [., Q]) for R rows; the outputs
+ * must not overlap the inputs. The backend's step past the last layer's attention, where only
+ * the rows with wanted logits go on (relay computes every row, cuda_backend.cu:575-595). */
+int rh_gather_rows(const float* x, int H, const void* a, int Q, const int* rows, int R, float* x_out, void* a_out,
+                   void* stream);
+
 /* Per token: qkv row += bias (if not NULL); RoPE on the q and k heads (pairs (i, i + D/2),
  * angle pos * inv_freq[i]); k and v written as fp16 into the paged cache; q written as
  * fp16(q * q_scale) to q_out (row stride heads * head_dim; may be NULL). q_scale = 1 is the

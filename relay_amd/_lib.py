@@ -102,6 +102,7 @@ SIGNATURES = {
     "rh_f32_to_f16": (I, [P, P, SZ, P]),
     "rh_embed": (I, [P, I, P, I, P, P]),
     "rh_rmsnorm": (I, [P, P, I, P, I, F, P, P]),
+    "rh_gather_rows": (I, [P, I, P, I, P, I, P, P, P]),
     "rh_qkv_post": (I, [P, I, P, P, P, P, P, P, P, P, P, F, I, I, I, I, P]),
     "rh_qkv_post_to_cache": (I, [P, I, P, P, P, P, P, P, P, P, P, F, I, I, I, I, P]),
     "rh_silu_mul": (I, [P, I, I, P, P]),

@@ -17,50 +17,12 @@
 // wave tiles); and the workgroups of an XCD cover a compact block of tiles (below).
 #include "../../include/relay_hip.h"
 #include "common.h"
+#include "lds_ring.h"
 
 #include <algorithm>
 
 namespace relay_hip {
 namespace {
-
-// ---- global memory -> LDS without registers -------------------------------------------
-//
-// buffer_load_dwordx4 ... lds: lane l's 16 bytes go to LDS address m0 + 16 l. Written as
-// asm because the builtin makes the compiler wait for vmcnt(0) before every LDS read it
-// cannot tell apart from the destination; here the ring's own waits (wait_vm) order them.
-// The instruction has no output register; every offset is clamped to the matrix.
-__device__ __forceinline__ uint4v f16_rsrc(const void* base) {
-  const uint64_t p = reinterpret_cast<uint64_t>(base);
-  return uint4v{static_cast<unsigned>(__builtin_amdgcn_readfirstlane(static_cast<int>(p))),
-                static_cast<unsigned>(__builtin_amdgcn_readfirstlane(static_cast<int>(p >> 32))) & 0xffffu,
-                0x7fffffffu, 0x00020000u};
-}
-
-__device__ __forceinline__ void load_to_lds(uint4v rsrc, uint32_t voffset, uint32_t soffset, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds"
-               :
-               : "v"(voffset), "s"(rsrc), "s"(soffset), "s"(lds)
-               : "memory");
-}
-
-// At most N of this wave's vector-memory operations still outstanding.
-template <int N>
-__device__ __forceinline__ void wait_vm() {
-  asm volatile("s_waitcnt vmcnt(%0)" : : "n"(N) : "memory");
-}
-
-// wait_vm<P * later> for later = min(later, MAX) (the count is an immediate).
-template <int P, int MAX>
-__device__ __forceinline__ void wait_stages(int later) {
-  if constexpr (MAX == 0) {
-    wait_vm<0>();
-  } else {
-    if (later >= MAX)
-      wait_vm<P * MAX>();
-    else
-      wait_stages<P, MAX - 1>(later);
-  }
-}
 
 constexpr int kMaxF16Split = 8;
 // Tiles are dealt to the XCDs as contiguous ranges (workgroup L runs on XCD L % 8) of an order
@@ -107,8 +69,8 @@ __global__ __launch_bounds__(WN * WT * WK * 64, 1) void gemm_f16_kernel(const ha
   // Lane l brings 16-byte chunk (l % 8) ^ swz(row) of row 8 p + l / 8: rows are stored with
   // their chunks XOR-permuted by (row >> 1) & 7, which makes the operand reads below cover
   // all 64 banks once per 16 lanes.
-  const uint4v wrs = f16_rsrc(w16);
-  const uint4v xrs = f16_rsrc(x);
+  const uint4v wrs = lds_rsrc(w16);
+  const uint4v xrs = lds_rsrc(x);
   uint32_t voff[LPS];
 #pragma unroll
   for (int i = 0; i < LPS; ++i) {
@@ -128,8 +90,7 @@ __global__ __launch_bounds__(WN * WT * WK * 64, 1) void gemm_f16_kernel(const ha
       voff[i] = static_cast<uint32_t>((static_cast<int64_t>(t) * K + ch * 8) * 2);
     }
   }
-  const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(
-      (__attribute__((address_space(3))) half_t*)lds));
+  const uint32_t lds0 = lds_address(lds);
   // Part `part` of `parts` of stage s's loads into ring buffer `buf`.
   auto issue = [&](int s, int buf, int part, int parts) {
     const uint32_t so = static_cast<uint32_t>((sbeg + s) * KS * 2);
@@ -172,8 +133,7 @@ __global__ __launch_bounds__(WN * WT * WK * 64, 1) void gemm_f16_kernel(const ha
   for (int s = 0; s < AHEAD; ++s)
     if (s < nsteps) issue(s, s, 0, 1);
   wait_stages<LPS, AHEAD - 1>(nsteps - 1);
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" : : : "memory");
+  ring_barrier();
   read(0, 0, 0);
   int buf = 0;
   for (int s = 0; s < nsteps; ++s) {
@@ -191,8 +151,7 @@ __global__ __launch_bounds__(WN * WT * WK * 64, 1) void gemm_f16_kernel(const ha
       // for all waves, and stage s's buffer takes stage s + STAGES.
       asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");
       wait_stages<LPS, STAGES - 2>(nsteps - 2 - s);
-      __builtin_amdgcn_s_barrier();
-      asm volatile("" : : : "memory");
+      ring_barrier();
       if (!SPREAD && s + STAGES < nsteps) issue(s + STAGES, buf, 0, 1);
       read(nbuf, 0, 0);
     }
@@ -203,8 +162,7 @@ __global__ __launch_bounds__(WN * WT * WK * 64, 1) void gemm_f16_kernel(const ha
     // Waves w and w + WN WT hold the two K halves of the same blocks: each keeps every other
     // block and hands the rest over through LDS.
     asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" : : : "memory");
+    ring_barrier();
     float* const xs = reinterpret_cast<float*>(lds) + (w % (WN * WT)) * (AN * AT * 1024) + lane * 4;
 #pragma unroll
     for (int i = 0; i < AN * AT; ++i)
@@ -215,8 +173,7 @@ __global__ __launch_bounds__(WN * WT * WK * 64, 1) void gemm_f16_kernel(const ha
               float4v{acc[i / AT][i % AT][4 * q], acc[i / AT][i % AT][4 * q + 1], acc[i / AT][i % AT][4 * q + 2],
                       acc[i / AT][i % AT][4 * q + 3]};
     asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" : : : "memory");
+    ring_barrier();
 #pragma unroll
     for (int i = 0; i < AN * AT; ++i)
       if ((i & 1) == wk)

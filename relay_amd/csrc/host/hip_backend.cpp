@@ -639,12 +639,16 @@ std::size_t HipBackend::enqueue_forward(const ForwardBatch& batch, LayerObserver
   const float q_scale = scale * 1.4426950408889634f, attn_scale = 0.6931471805599453f;
   HIP_CHECK(hipEventRecord(fwd_begin_, stream_));
   RH_CHECK(rh_embed(d_tok, T, embed_.p, H, x_.p, stream_));
+  // The rows of the residual stream after attention: all T, in the last layer the wanted ones.
+  int Tl = T;
+  float* xl = x_.p;
+  const std::uint16_t* al = attn_.p;
   // x += the product whose ks partials are in split_ws_, xn = its RMSNorm.
-  auto merge_rmsnorm = [&](const DeviceMatrix& W, int ks, int rows, const float* norm) {
+  auto merge_rmsnorm = [&](const DeviceMatrix& W, int ks, const float* norm) {
     if (W.i8.p)
-      RH_CHECK(rh_w8_merge_rmsnorm(split_ws_.p, ks, rows, H, W.scale.p, x_.p, norm, eps, xn_.p, stream_));
+      RH_CHECK(rh_w8_merge_rmsnorm(split_ws_.p, ks, Tl, H, W.scale.p, xl, norm, eps, xn_.p, stream_));
     else
-      RH_CHECK(rh_f16_merge_rmsnorm(split_ws_.p, ks, rows, H, x_.p, norm, eps, xn_.p, stream_));
+      RH_CHECK(rh_f16_merge_rmsnorm(split_ws_.p, ks, Tl, H, xl, norm, eps, xn_.p, stream_));
   };
   bool attn_xn_ready = false;  // the previous layer's fused down merge wrote this layer's xn
   for (int l = 0; l < c_.layers; ++l) {
@@ -713,77 +717,87 @@ std::size_t HipBackend::enqueue_forward(const ForwardBatch& batch, LayerObserver
       RH_CHECK(rh_reference_attention(qkv_.p, QKV, kc, vc, d_pos, d_seq, d_toff, d_tab, nullptr, T, c_.heads,
                                       c_.kv_heads, D, layout_.block_size, scale, attn_.p, Q, stream_));
     }
+    // Past the last layer's attention only the rows whose logits are wanted matter: they move
+    // together (into the qkv and query buffers, free by now) and the rest of the pass runs on
+    // them alone, a 512-token prompt chunk on one row.
+    if (l + 1 == c_.layers && R < T && H <= QKV) {
+      if (!R) break;
+      RH_CHECK(rh_gather_rows(x_.p, H, attn_.p, Q, d_rows, R, qkv_.p, qh_.p, stream_));
+      Tl = R;
+      xl = qkv_.p;
+      al = qh_.p;
+    }
     // int8 products split over K (17+ tokens) leave their partials to the consumer: the o
     // and down projections' merge, residual add and following RMSNorm run as one launch,
     // the gate_up merge and SiLU as another (TinyLlama int8 32 x 2048 decode step: two
     // launches fewer per layer).
     bool mlp_xn_ready = false;
     const bool merge_norm = rh_w8_merge_rmsnorm_fits(H);
-    if (const int ks = merge_norm ? partials(L.wo, attn_.p, T) : 0) {
-      merge_rmsnorm(L.wo, ks, T, L.mlp_norm.p);
+    if (const int ks = merge_norm ? partials(L.wo, al, Tl) : 0) {
+      merge_rmsnorm(L.wo, ks, L.mlp_norm.p);
       mlp_xn_ready = true;
     } else {
-      gemm(L.wo, attn_.p, x_.p, T, 1.0f);  // x += attn W_o^T
+      gemm(L.wo, al, xl, Tl, 1.0f);  // x += attn W_o^T
     }
     bool act_ready = false;
-    if (fused(L.w_gate_up, T)) {
-      RH_CHECK(rh_gemv_f16_rmsnorm(L.w_gate_up.f16.p, H, x_.p, L.mlp_norm.p, eps, gu_.p, T, H, 2 * I, 0.0f,
+    if (fused(L.w_gate_up, Tl)) {
+      RH_CHECK(rh_gemv_f16_rmsnorm(L.w_gate_up.f16.p, H, xl, L.mlp_norm.p, eps, gu_.p, Tl, H, 2 * I, 0.0f,
                                    stream_));
     } else {
       // (int8 at 9-16 tokens: level at b = 12, 1.29 -> 1.305 ms at b = 16 on TinyLlama.)
-      const bool i8_silu = L.w_gate_up.i8.p && T <= 8 && H % 16 == 0;
+      const bool i8_silu = L.w_gate_up.i8.p && Tl <= 8 && H % 16 == 0;
       // fp16 where gemm() would take the whole-line product: the same kernel with SiLU·mul
       // in its epilogue.
-      const bool f16_silu = !L.w_gate_up.i8.p && skinny(H, 2 * I, T) && T <= 32;
-      if (i8_silu && !mlp_xn_ready && rh_gemv_f16_fused_fits(T, H) && (I + 7) / 8 < 256) {
+      const bool f16_silu = !L.w_gate_up.i8.p && skinny(H, 2 * I, Tl) && Tl <= 32;
+      if (i8_silu && !mlp_xn_ready && rh_gemv_f16_fused_fits(Tl, H) && (I + 7) / 8 < 256) {
         // The RMSNorm, the int8 product and SiLU·mul in one launch, where its workgroups
         // (8 outputs each) fit one round on the CUs: every workgroup normalises x again, which
         // at more rounds costs more than the launch it saves (SmolLM2-135M int8 decode, 192
         // workgroups: 0.770 -> 0.733 ms per step; TinyLlama, 704: 0.854 -> 0.968).
-        RH_CHECK(rh_gemv_int8_rmsnorm_gate_up_silu(L.w_gate_up.i8.p, L.w_gate_up.ldw, L.w_gate_up.scale.p, 0, x_.p,
-                                                   L.mlp_norm.p, eps, act_.p, T, H, I, stream_));
+        RH_CHECK(rh_gemv_int8_rmsnorm_gate_up_silu(L.w_gate_up.i8.p, L.w_gate_up.ldw, L.w_gate_up.scale.p, 0, xl,
+                                                   L.mlp_norm.p, eps, act_.p, Tl, H, I, stream_));
         act_ready = true;
       } else {
-        if (!mlp_xn_ready) RH_CHECK(rh_rmsnorm(x_.p, nullptr, T, L.mlp_norm.p, H, eps, xn_.p, stream_));
+        if (!mlp_xn_ready) RH_CHECK(rh_rmsnorm(xl, nullptr, Tl, L.mlp_norm.p, H, eps, xn_.p, stream_));
         // Above 64 tokens, where the plan runs gate_up unsplit on the 256 x 96 tile: the same
         // product with SiLU·mul in its epilogue (same bytes, no fp32 [T, 2 I] round trip).
-        const bool tile_silu = L.w_gate_up.i8.p && T > 64 && rh_gemm_w8_plan(T, H, 2 * I) == 1 &&
-                               rh_gemm_w8_kernel(T, H, 2 * I, 1) == 1 &&
+        const bool tile_silu = L.w_gate_up.i8.p && Tl > 64 && rh_gemm_w8_plan(Tl, H, 2 * I) == 1 &&
+                               rh_gemm_w8_kernel(Tl, H, 2 * I, 1) == 1 &&
                                (static_cast<std::int64_t>(I) + 256) * L.w_gate_up.ldw < (std::int64_t(1) << 31);
         // fp16 above the whole-line kernel's range: SiLU·mul in the tile kernel's epilogue. On
         // products large enough for the library that saves the fp32 [T, 2 I] round trip and
         // a launch, which outweighs the library's faster kernel while K is short (2048 tokens
         // of TinyLlama: 104 us against 97 + 22; 512 of Llama-3-8B: 130 against 106 + 12).
-        const bool f16_tile = !L.w_gate_up.i8.p && !skinny(H, 2 * I, T) &&
-                              (tiled(H, 2 * I, T) || (H <= 2048 && rh_gemm_f16_fits(T, H, 2 * I)));
-        const int ks = tile_silu || f16_tile || I % 8 ? 0 : w8_partials(L.w_gate_up, xn_.p, T);
+        const bool f16_tile = !L.w_gate_up.i8.p && !skinny(H, 2 * I, Tl) &&
+                              (tiled(H, 2 * I, Tl) || (H <= 2048 && rh_gemm_f16_fits(Tl, H, 2 * I)));
+        const int ks = tile_silu || f16_tile || I % 8 ? 0 : w8_partials(L.w_gate_up, xn_.p, Tl);
         if (f16_tile) {
-          const int gks = rh_gemm_f16_gate_up_plan(T, H, I);
+          const int gks = rh_gemm_f16_gate_up_plan(Tl, H, I);
           if (gks > 1) {
-            RH_CHECK(rh_gemm_f16_partials(L.w_gate_up.f16.p, H, xn_.p, T, H, 2 * I, gks, w8_split_ws(gks, T, 2 * I), stream_));
-            RH_CHECK(rh_f16_merge_silu(split_ws_.p, gks, T, I, act_.p, stream_));
+            RH_CHECK(rh_gemm_f16_partials(L.w_gate_up.f16.p, H, xn_.p, Tl, H, 2 * I, gks, w8_split_ws(gks, Tl, 2 * I), stream_));
+            RH_CHECK(rh_f16_merge_silu(split_ws_.p, gks, Tl, I, act_.p, stream_));
           } else {
-            RH_CHECK(rh_gemm_f16_gate_up_silu(L.w_gate_up.f16.p, H, xn_.p, act_.p, T, H, I, stream_));
+            RH_CHECK(rh_gemm_f16_gate_up_silu(L.w_gate_up.f16.p, H, xn_.p, act_.p, Tl, H, I, stream_));
           }
           act_ready = true;
         } else if (tile_silu) {
-          RH_CHECK(rh_gemm_w8_gate_up_silu(L.w_gate_up.i8.p, L.w_gate_up.ldw, L.w_gate_up.scale.p, xn_.p, act_.p, T, H,
+          RH_CHECK(rh_gemm_w8_gate_up_silu(L.w_gate_up.i8.p, L.w_gate_up.ldw, L.w_gate_up.scale.p, xn_.p, act_.p, Tl, H,
                                            I, stream_));
           act_ready = true;
         } else if (ks) {
-          RH_CHECK(rh_w8_merge_silu(split_ws_.p, ks, T, I, L.w_gate_up.scale.p, act_.p, stream_));
+          RH_CHECK(rh_w8_merge_silu(split_ws_.p, ks, Tl, I, L.w_gate_up.scale.p, act_.p, stream_));
           act_ready = true;
         } else if (i8_silu) {
           // gemm()'s product at this T (the int8 GEMV) with SiLU·mul in its epilogue: one
           // launch fewer per layer (the same bits at 1-8 tokens).
           RH_CHECK(rh_gemv_int8_gate_up_silu(L.w_gate_up.i8.p, L.w_gate_up.ldw, L.w_gate_up.scale.p, 0, xn_.p,
-                                             act_.p, T, H, I, stream_));
+                                             act_.p, Tl, H, I, stream_));
           act_ready = true;
         } else if (f16_silu) {
-          RH_CHECK(rh_gemv_f16_gate_up_silu(L.w_gate_up.f16.p, H, xn_.p, act_.p, T, H, I, stream_));
+          RH_CHECK(rh_gemv_f16_gate_up_silu(L.w_gate_up.f16.p, H, xn_.p, act_.p, Tl, H, I, stream_));
           act_ready = true;
         } else {
-          gemm(L.w_gate_up, xn_.p, gu_.p, T, 0.0f);
+          gemm(L.w_gate_up, xn_.p, gu_.p, Tl, 0.0f);
         }
       }
     }
@@ -791,22 +805,22 @@ std::size_t HipBackend::enqueue_forward(const ForwardBatch& batch, LayerObserver
     // small (TinyLlama fp16 decode, I = 5632: b = 2 1.085 -> 1.063 ms, b = 4 1.177 -> 1.103
     // with the separate SiLU launch, level at b = 1 and 8; SmolLM2-135M, I = 1536, b = 1
     // fused: 1087 against 1048 tok/s).
-    if (!act_ready && fused(L.w_down, T) && T * I <= 8192) {
-      RH_CHECK(rh_gemv_f16_silu(L.w_down.f16.p, I, gu_.p, x_.p, T, I, H, 1.0f, stream_));  // x += act W_down^T
+    if (!act_ready && fused(L.w_down, Tl) && Tl * I <= 8192) {
+      RH_CHECK(rh_gemv_f16_silu(L.w_down.f16.p, I, gu_.p, xl, Tl, I, H, 1.0f, stream_));  // x += act W_down^T
     } else {
-      if (!act_ready) RH_CHECK(rh_silu_mul(gu_.p, T, I, act_.p, stream_));
-      const int ks = merge_norm ? partials(L.w_down, act_.p, T) : 0;
+      if (!act_ready) RH_CHECK(rh_silu_mul(gu_.p, Tl, I, act_.p, stream_));
+      const int ks = merge_norm ? partials(L.w_down, act_.p, Tl) : 0;
       if (ks) {  // x += act W_down^T, then the next layer's attention RMSNorm (or the final one)
-        merge_rmsnorm(L.w_down, ks, T, l + 1 < c_.layers ? layers_[l + 1].attn_norm.p : final_norm_.p);
+        merge_rmsnorm(L.w_down, ks, l + 1 < c_.layers ? layers_[l + 1].attn_norm.p : final_norm_.p);
         attn_xn_ready = true;
       } else {
-        gemm(L.w_down, act_.p, x_.p, T, 1.0f);  // x += act W_down^T
+        gemm(L.w_down, act_.p, xl, Tl, 1.0f);  // x += act W_down^T
       }
     }
   }
   if (R) {
     // The last merge wrote the final norm of every row: of the wanted ones when all are.
-    if (!(attn_xn_ready && R == T)) RH_CHECK(rh_rmsnorm(x_.p, d_rows, R, final_norm_.p, H, eps, xn_.p, stream_));
+    if (!(attn_xn_ready && R == Tl)) RH_CHECK(rh_rmsnorm(xl, R == Tl ? nullptr : d_rows, R, final_norm_.p, H, eps, xn_.p, stream_));
     gemm_f16(lm_head_.n ? lm_head_.p : embed_.p, xn_.p, logits_.p, R, H, V, 0.0f);
   }
   HIP_CHECK(hipEventRecord(fwd_end_, stream_));

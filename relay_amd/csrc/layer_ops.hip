@@ -133,6 +133,15 @@ __global__ void rmsnorm_vec_kernel(const float* x, const int* rows, const float*
   }
 }
 
+// x_out[r] = x[rows[r]] (H floats), a_out[r] = a[rows[r]] (Q halves): the rows that go on past the
+// last attention. One workgroup per row; bound by its launch (3 us for 49 rows of 4096).
+__global__ void gather_rows_kernel(const float* x, int H, const half_t* a, int Q, const int* rows, float* x_out,
+                                   half_t* a_out) {
+  const int64_t r = blockIdx.x, from = rows[r];
+  for (int i = threadIdx.x; i < H; i += kThreads) x_out[r * H + i] = x[from * H + i];
+  for (int i = threadIdx.x; i < Q; i += kThreads) a_out[r * Q + i] = a[from * Q + i];
+}
+
 // ---- the K-range merge of a split product, fused into its consumer ----------------------
 //
 // rh_gemm_w8_partials and rh_gemm_f16_partials leave ksn raw partial planes ws[z][t][n] (fp16
@@ -534,6 +543,16 @@ int rh_rmsnorm(const float* x, const int* rows, int R, const float* w, int H, fl
                    (reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(out)) % 16 == 0;
   RH_TRY_LAUNCH(hipLaunchKernelGGL(vec ? rmsnorm_vec_kernel : rmsnorm_kernel, dim3(R), dim3(kThreads), 0,
                                    static_cast<hipStream_t>(stream), x, rows, w, H, eps, static_cast<half_t*>(out)));
+  return 0;
+}
+
+int rh_gather_rows(const float* x, int H, const void* a, int Q, const int* rows, int R, float* x_out, void* a_out,
+                   void* stream) {
+  if (R == 0) return 0;
+  RH_REQUIRE(R > 0 && H > 0 && Q > 0, "gather_rows: bad shape");
+  RH_REQUIRE(x && a && rows && x_out && a_out && x != x_out && a != a_out, "gather_rows: bad pointer");
+  RH_TRY_LAUNCH(hipLaunchKernelGGL(gather_rows_kernel, dim3(R), dim3(kThreads), 0, static_cast<hipStream_t>(stream), x, H,
+                                   static_cast<const half_t*>(a), Q, rows, x_out, static_cast<half_t*>(a_out)));
   return 0;
 }
 

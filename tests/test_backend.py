@@ -273,3 +273,32 @@ def test_read_kv_layer_into_a_caller_buffer(dev):
     with pytest.raises(ValueError):
         be.read_kv_layer(1, blocks, out=np.empty(fresh.size - 1, np.uint8))
     be.close()
+
+
+@pytest.mark.parametrize("int8", [False, True])
+def test_rows_without_logits_are_dropped_after_the_last_attention(dev, int8):
+    """A batch in which some chunks want no logits: the wanted rows agree with the same rows of
+    an all-logits pass, and the KV cache holds the same bytes, so that a pass that wants none at
+    all leaves the next one unchanged."""
+    w = small_model(64, 8, 2, layers=3, hidden=512, inter=768)
+    opts = HipOptions(False, int8)
+    a, b = HipBackend(w, 40, 16, options=opts), HipBackend(w, 40, 16, options=opts)
+    rng = np.random.default_rng(5)
+    tab = [list(range(20)), list(range(20, 30)), list(range(30, 40))]
+    prompts = [rng.integers(0, 512, n).tolist() for n in (130, 40, 7)]
+
+    def batch(wants, everything=False):
+        return ForwardBatch([SeqChunk(p, 0, t, x) for p, t, x in zip(prompts, tab, wants)], all_logits=everything)
+
+    full = a.forward(batch([True] * 3, everything=True))
+    last = np.cumsum([len(p) for p in prompts]) - 1
+    for wants in ([False, True, True], [True, False, False], [False, False, False], [True, True, True]):
+        got = b.forward(batch(wants))
+        want = full[last[np.array(wants)]]
+        assert got.shape == want.shape
+        if len(want):
+            assert rel_err_rowmax(got, want) < 2e-3
+        for layer in range(3):
+            assert np.array_equal(a.read_kv_layer(layer, list(range(40))), b.read_kv_layer(layer, list(range(40))))
+    step = lambda be: be.forward(ForwardBatch([SeqChunk([7], len(p), t, True) for p, t in zip(prompts, tab)]))
+    assert np.array_equal(step(a), step(b))

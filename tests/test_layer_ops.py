@@ -301,3 +301,20 @@ def test_qkv_post_to_cache_matches_qkv_post(torch_mod, dev, bs):
     assert _lib.lib().rh_qkv_post_to_cache(None, 1, None, None, None, None, None, None, None, None, None, 1.0, 8, 2, 64,
                                            16, None) != 0
     assert "q_out is required" in _lib.last_error()
+
+
+def test_gather_rows(torch_mod, dev):
+    """Rows in any order, widths that are no multiple of the workgroup; the rest stays."""
+    from relay_amd import _lib
+
+    L = _lib.lib()
+    rng = np.random.default_rng(11)
+    x, a = rng.standard_normal((9, 577)).astype(np.float32), rng.integers(0, 1 << 15, (9, 1030)).astype(np.int16)
+    rows = np.array([8, 0, 3], np.int32)
+    X, A, R = (torch_mod.from_numpy(v).to(dev) for v in (x, a, rows))
+    xo, ao = torch_mod.full((4, 577), 5.0, device=dev), torch_mod.full((4, 1030), 5, dtype=torch_mod.int16, device=dev)
+    _lib.check(L.rh_gather_rows(X.data_ptr(), 577, A.data_ptr(), 1030, R.data_ptr(), 3, xo.data_ptr(), ao.data_ptr(), None))
+    torch_mod.cuda.synchronize()
+    assert np.array_equal(xo.cpu().numpy()[:3], x[rows]) and np.array_equal(ao.cpu().numpy()[:3], a[rows])
+    assert (xo[3] == 5.0).all() and (ao[3] == 5).all()
+    assert L.rh_gather_rows(X.data_ptr(), 577, A.data_ptr(), 1030, R.data_ptr(), 3, X.data_ptr(), ao.data_ptr(), None) != 0
