@@ -95,7 +95,8 @@ struct Stage {
 // size 16, which runs at width 32 with dims 16..31 of K, V and q taken as zero.
 // Occupancy: up to D = 64 the kernel fits 128 VGPRs, so a CU holds two 8-wave workgroups
 // (4 waves per SIMD); at D = 128 it needs more and holds one.
-template <int D, int DR, int WAVES, bool SCALAR>
+// BY_PART: the order of the slices over the workgroups (below).
+template <int D, int DR, int WAVES, bool SCALAR, bool BY_PART>
 __global__ __launch_bounds__(WAVES * kWave) __attribute__((amdgpu_waves_per_eu(D <= 64 ? 4 : 2, D <= 64 ? 4 : 2))) void paged_decode_kernel(
     const DecodeArgs a) {
   constexpr int SK = stage_keys<D>();
@@ -117,11 +118,14 @@ __global__ __launch_bounds__(WAVES * kWave) __attribute__((amdgpu_waves_per_eu(D
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int c = lane & 15, g = lane >> 4;
 
-  // Workgroup -> (group, part), the slices of one group on one XCD.
+  // Workgroup -> (group, part), the slices of one group on one XCD. A launch of several rounds
+  // takes every group's last slice first, then the ones before it: the long contexts' slices
+  // start early and the ends of shorter ones, which exit at once, are spread over the CUs (with
+  // a group's slices side by side they fell on the same CUs wherever max_parts divides 32).
   const int b = blockIdx.x;
-  const int sl = b >> 3;
-  const int part = sl % a.max_parts;
-  const int grp = (sl / a.max_parts) * 8 + (b & 7);
+  const int sl = b >> 3, run = BY_PART ? (a.groups_total + 7) >> 3 : a.max_parts;
+  const int part = BY_PART ? a.max_parts - 1 - sl / run : sl % run;
+  const int grp = (BY_PART ? sl % run : sl / run) * 8 + (b & 7);
   if (grp >= a.groups_total) return;
   const int per_tok = a.kv_heads * a.hchunks;
   const int di = grp / per_tok;
@@ -424,21 +428,26 @@ __global__ __launch_bounds__(WAVES * kWave) __attribute__((amdgpu_waves_per_eu(D
   }
 }
 
-template <int D, int DR, int WAVES>
-int launch(const DecodeArgs& a, int grid, hipStream_t s) {
-  if (a.bs_shift >= 4) {
-    RH_TRY_LAUNCH(
-        hipLaunchKernelGGL((paged_decode_kernel<D, DR, WAVES, true>), dim3(grid), dim3(WAVES * kWave), 0, s, a));
+template <int D, int DR, int WAVES, bool SCALAR>
+int launch(const DecodeArgs& a, int grid, bool by_part, hipStream_t s) {
+  if (by_part) {
+    RH_TRY_LAUNCH(hipLaunchKernelGGL((paged_decode_kernel<D, DR, WAVES, SCALAR, true>), dim3(grid), dim3(WAVES * kWave), 0, s, a));
   } else {
-    RH_TRY_LAUNCH(
-        hipLaunchKernelGGL((paged_decode_kernel<D, DR, WAVES, false>), dim3(grid), dim3(WAVES * kWave), 0, s, a));
+    RH_TRY_LAUNCH(hipLaunchKernelGGL((paged_decode_kernel<D, DR, WAVES, SCALAR, false>), dim3(grid), dim3(WAVES * kWave), 0, s, a));
   }
   return 0;
 }
 
 template <int D, int DR>
 int launch_waves(const DecodeArgs& a, int grid, bool eight, hipStream_t s) {
-  return eight ? launch<D, DR, 8>(a, grid, s) : launch<D, DR, 4>(a, grid, s);
+  // Workgroups on the chip at a time: two per CU up to head size 64, one at 128. Measured (us,
+  // side by side / by part; contexts random in [ctx / 8, ctx]): 48 x 8192, 32/8 heads, D128 183.8 /
+  // 167.8, 48 x 2048 62.5 / 55.0, 48 x 8192, 9/3, D64, 1024-key slices 36.6 / 35.2; equal contexts
+  // level. In one round a group's slices end together side by side: 32 x 2048, 32/4, D64 12.4 / 13.1.
+  const bool by_part = grid > (D <= 64 ? 512 : 256);
+  if (a.bs_shift >= 4)
+    return eight ? launch<D, DR, 8, true>(a, grid, by_part, s) : launch<D, DR, 4, true>(a, grid, by_part, s);
+  return eight ? launch<D, DR, 8, false>(a, grid, by_part, s) : launch<D, DR, 4, false>(a, grid, by_part, s);
 }
 
 }  // namespace
@@ -477,7 +486,18 @@ extern "C" int rh_decode_slice_keys(int n_dec, int kv_heads, int group, int head
   }
   // A handful of short contexts: one slice (no merge); the launch is latency-bound anyway.
   if (groups <= 16 && max_ctx <= 16 * chunk) return (max_ctx + chunk - 1) / chunk * chunk;
-  const long parts = std::max(2L, 256 / groups);
+  long parts = std::max(2L, 256 / groups);
+  // Past one workgroup per CU with two slices: the fewest slices that fill whole rounds of 256
+  // workgroups to 85% (else the fullest). Measured (us, 2 slices / these): 144 groups, 9/3 heads,
+  // D64, 8192 keys 68.5 / 52 (ragged 54 / 37), 192 groups, 32/4, D64, 4096 keys 42.5 / 38.1 (ragged 31.2 /
+  // 23.9); 384 groups fill three rounds with two.
+  if (groups > 128) {
+    double best = 0.0;
+    for (long p = 2; p <= kMergeBatch && best < 0.85; ++p) {
+      const double fill = static_cast<double>(groups * p) / ((groups * p + 255) / 256 * 256);
+      if (fill > best) best = fill, parts = p;
+    }
+  }
   const long per_part = (max_ctx + parts - 1) / parts;
   const long keys = std::max(8L * chunk, (per_part + chunk - 1) / chunk * chunk);
   return static_cast<int>(keys);

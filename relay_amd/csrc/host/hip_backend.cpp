@@ -205,11 +205,12 @@ class HipBackend final : public Backend {
   // copied on to dst as soon as it lands, under the DMA of the next.
   void finish_forward(float* dst, std::size_t n);
   static constexpr int kLogitChunks = 16;
-  // Each D2H piece costs ~10 us of its own beyond its bytes: TinyLlama's 4 MB of logits for
-  // 32 rows took 0.43 ms from the forward's end to the caller's buffer in 16 pieces of 256
-  // KB, 0.29 ms in 4 of 1 MB (one piece then 4 threads: 0.33 ms); 25 MB in 16 pieces level.
-  static constexpr std::size_t kLogitMinPiece = std::size_t(1) << 20;
-  static constexpr int kLogitThreads = 4;
+  // Each D2H piece costs ~10 us of its own beyond its bytes, each helper thread ~15 us to start.
+  // Whole steps with 4.1 / 6.3 MB of logits (us): 256 KB pieces on 3 threads 646 / 1065, 512 KB 533 /
+  // 1007, 1 MB 475 / 929, 2 MB 456 / 907, 4 MB 490 / 915; 2 MB on 1, 2, 4, 6 threads 506, 459, 458, 497 /
+  // 974, 912, 909, 944.
+  static constexpr std::size_t kLogitMinPiece = std::size_t(2) << 20;
+  static constexpr int kLogitThreads = 3;
   static constexpr std::size_t kLogitThreadBytes = std::size_t(2) << 20;
   std::vector<hipEvent_t> logit_events_;
   // Set while a pass without an observer runs. Only an observed pass records layer_done_ events

@@ -225,3 +225,18 @@ def test_slice_merge_is_stable_over_many_launches(torch_mod, dev):
     torch.cuda.synchronize()
     assert int(bad.item()) == 0, f"{int(bad.item())} of 300 launches differed from the first"
     assert int(ctr.abs().sum().item()) == 0
+
+
+@pytest.mark.parametrize("D,slice_keys,bs", [(16, 128, 16), (64, 64, 16), (64, 128, 12), (128, 64, 16), (128, 32, 5)])
+@pytest.mark.parametrize("n", [11, 40])
+def test_slices_of_several_rounds(torch_mod, dev, D, slice_keys, bs, n):
+    """Launches of more workgroups than the chip holds at a time (512, at head size 128 256) take
+    every context's last slices first: ragged contexts, a slice of one key, contexts of one
+    slice beside one of many; a group count that is no multiple of the 8 XCDs; the counters
+    come back zero."""
+    rng = np.random.default_rng(D + n)
+    ctx = rng.integers(1, 700, size=n).tolist() + [1, slice_keys, slice_keys + 1, 2900]
+    case = PagedCase(ctx, 1, 9, 3, D, bs, seed=D + n)
+    g, counters = run_decode(torch_mod, dev, case, slice_keys=slice_keys)
+    check_close(g, oracle_out(case))
+    assert not counters.any()
