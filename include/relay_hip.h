@@ -448,6 +448,13 @@ int rh_kv_gather(const void* kpool, const void* vpool, const int* blocks, int n,
 int rh_kv_scatter(void* kpool, void* vpool, const int* blocks, int n, size_t block_bytes, const void* buf,
                   void* stream);
 
+/* The same with buf in pinned host memory that the device can address, on few workgroups (PCIe
+ * is the bound, and a transfer should leave the CUs to the pass that runs beside it). */
+int rh_kv_gather_to_host(const void* kpool, const void* vpool, const int* blocks, int n, size_t block_bytes, void* buf,
+                         void* stream);
+int rh_kv_scatter_from_host(void* kpool, void* vpool, const int* blocks, int n, size_t block_bytes, const void* buf,
+                            void* stream);
+
 /* Fills out[i] (i < n) with fp16 / fp32 draws of mean + std * N(0, 1) from the
  * counter-based generator of rh_synth_normal_f32 (seed, stream, counter i). */
 int rh_fill_normal_f16(void* out, size_t n, uint64_t seed, uint64_t stream_id, float mean, float std, void* stream);

@@ -108,6 +108,8 @@ SIGNATURES = {
     "rh_silu_mul": (I, [P, I, I, P, P]),
     "rh_kv_gather": (I, [P, P, P, I, SZ, P, P]),
     "rh_kv_scatter": (I, [P, P, P, I, SZ, P, P]),
+    "rh_kv_gather_to_host": (I, [P, P, P, I, SZ, P, P]),
+    "rh_kv_scatter_from_host": (I, [P, P, P, I, SZ, P, P]),
     "rh_fill_normal_f16": (I, [P, SZ, U64, U64, F, F, P]),
     "rh_fill_normal_f32": (I, [P, SZ, U64, U64, F, F, P]),
     "rh_synth_normal_f32": (None, [P, SZ, U64, U64, F, F]),

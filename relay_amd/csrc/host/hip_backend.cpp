@@ -253,13 +253,17 @@ class HipBackend final : public Backend {
   // Whether gemm_f16 runs the skinny product (else the library GEMM) for this shape.
   static bool skinny(int K, int N, int T);
   void kv_io(int layer, const std::vector<int>& blocks, void* k_out, void* v_out, const void* k_in, const void* v_in);
-  // Pieces of one KV transfer: writes in up to 16, reads in up to 8 (each DMA piece costs
-  // ~10 us beyond its bytes, and a read's host copies are split over the threads; Llama-3
-  // layer reads of 33.6 MB: 34.1 GB/s at 16 pieces, 36.9-38.8 at 8, 38.5-39.1 at 4, 28-31 at 2;
-  // writes 35.5 at 16, 34-36 at 8, 30.5 at 4).
-  static constexpr int kKvChunks = 16, kKvReadChunks = 8;
-  static constexpr int kKvThreads = 4;                          // host threads copying them (8: no faster)
-  static constexpr std::size_t kKvMinPiece = std::size_t(1) << 20;
+  // Pieces of a large KV transfer: writes in 16, reads in 8 (each DMA piece costs ~10 us beyond
+  // its bytes, and a read's host copies are split over the threads; Llama-3 layer reads of 33.6
+  // MB: 34.1 GB/s at 16 pieces, 36.9-38.8 at 8, 38.5-39.1 at 4, 28-31 at 2; writes 35.5 at 16,
+  // 34-36 at 8, 30.5 at 4). Up to 8 MB kernels read and write the pinned staging buffer
+  // themselves, in up to 16 pieces of at least 512 KB: no device copy and no DMA set-up per piece
+  // (4.2 MB: write 125 -> 92 us, read 112 -> 92; 0.5 MB: 50 -> 34, 55 -> 38; at 33.6 MB level within
+  // the runs' spread, writes 870 by DMA, 960-1020 by kernels).
+  static constexpr int kKvPieces = 16, kKvReadPieces = 8;
+  static constexpr std::size_t kKvDirect = std::size_t(8) << 20;
+  static constexpr int kKvThreads = 4;  // host threads copying them (8: no faster)
+  static constexpr std::size_t kKvMinPiece = std::size_t(512) << 10;
   std::vector<hipEvent_t> kv_events_;                           // one per piece in flight
 
   ModelConfig c_;
@@ -950,11 +954,9 @@ void HipBackend::finish_forward(float* dst, std::size_t n) {
   });
 }
 
-// KV block traffic on the copy stream: gather into a contiguous device buffer and copy it
-// to pinned host memory (and the reverse for writes), in pieces so that the host-side
-// memcpy of one piece runs under the DMA of the next (one Llama-3-8B layer at 8192
-// positions, 33.6 MB, into and out of caller buffers: one piece 10.9 / 20.8 GB/s read /
-// write, pieces on one host thread 26.4 / 30.5, now ~37 / ~36). Serialised by copy_mu_.
+// KV block traffic on the copy stream, between the cache and pinned host memory, in pieces so
+// that the host-side memcpy of one piece runs under the transfer of the next. Serialised by
+// copy_mu_.
 void HipBackend::kv_io(int layer, const std::vector<int>& blocks, void* k_out, void* v_out, const void* k_in,
                        const void* v_in) {
   if (layer < 0 || layer >= c_.layers) throw std::invalid_argument("layer out of range");
@@ -964,7 +966,6 @@ void HipBackend::kv_io(int layer, const std::vector<int>& blocks, void* k_out, v
   if (!n) return;
   std::lock_guard<std::mutex> lock(copy_mu_);
   const std::size_t bytes = 2 * n * bb;
-  if (kv_stage_dev_.n < bytes) kv_stage_dev_ = DeviceArray<unsigned char>(bytes);
   if (kv_ids_dev_.n < n) kv_ids_dev_ = DeviceArray<int>(n);
   kv_stage_host_.reserve(bytes + n * sizeof(int));
   auto* host = static_cast<unsigned char*>(kv_stage_host_.p);
@@ -973,59 +974,103 @@ void HipBackend::kv_io(int layer, const std::vector<int>& blocks, void* k_out, v
   HIP_CHECK(hipMemcpyAsync(kv_ids_dev_.p, ids, n * sizeof(int), hipMemcpyHostToDevice, copy_stream_));
   const std::size_t off = static_cast<std::size_t>(layer) * layout_.layer_elems();
   if (kv_events_.empty()) {
-    kv_events_.resize(kKvChunks);
+    kv_events_.resize(kKvPieces);
     for (auto& e : kv_events_) HIP_CHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
   }
-  // Staging bytes [0, n bb) are K, [n bb, 2 n bb) V; piece i covers [i piece, (i+1) piece).
-  const int chunks = k_out ? kKvReadChunks : kKvChunks;
-  const std::size_t piece = std::max<std::size_t>(kKvMinPiece, (bytes + chunks - 1) / chunks);
-  const int pieces = static_cast<int>((bytes + piece - 1) / piece);
   // The host-side copies between the caller's buffers and the pinned staging run on a few
-  // threads (one core moves ~10-25 GB/s; the DMA runs at the PCIe rate).
-  const int workers = bytes >= kLogitThreadBytes ? std::min(kKvThreads, pieces) : 1;
-  auto user_copy = [&](std::size_t a, std::size_t len, bool to_user) {
-    // [a, a + len) of the staging buffer to / from k_out|k_in and v_out|v_in.
-    while (len) {
-      const bool is_k = a < n * bb;
-      const std::size_t rel = is_k ? a : a - n * bb, take = std::min(len, n * bb - rel);
-      auto* u = static_cast<unsigned char*>(is_k ? (to_user ? k_out : const_cast<void*>(k_in))
-                                                 : (to_user ? v_out : const_cast<void*>(v_in)));
-      if (to_user) std::memcpy(u + rel, host + a, take);
-      else std::memcpy(host + a, u + rel, take);
-      a += take;
-      len -= take;
+  // threads (one core moves ~10-25 GB/s; the transfers run at the PCIe rate).
+  const int workers = bytes >= kLogitThreadBytes ? kKvThreads : 1;
+  if (bytes > kKvDirect) {
+    // Staging bytes [0, n bb) are K, [n bb, 2 n bb) V, here and on the device; the DMA engine
+    // moves them in pieces, piece i [i piece, (i + 1) piece).
+    if (kv_stage_dev_.n < bytes) kv_stage_dev_ = DeviceArray<unsigned char>(bytes);
+    const int chunks = k_out ? kKvReadPieces : kKvPieces;
+    const std::size_t piece = (bytes + chunks - 1) / chunks;
+    const int pieces = static_cast<int>((bytes + piece - 1) / piece);
+    auto user_copy = [&](std::size_t from, std::size_t to, bool to_user) {
+      for (int v = 0; v < 2; ++v) {
+        const std::size_t lo = std::max(from, v * n * bb), hi = std::min(to, (v + 1) * n * bb);
+        if (lo >= hi) continue;
+        if (to_user)
+          std::memcpy(static_cast<unsigned char*>(v ? v_out : k_out) + (lo - v * n * bb), host + lo, hi - lo);
+        else
+          std::memcpy(host + lo, static_cast<const unsigned char*>(v ? v_in : k_in) + (lo - v * n * bb), hi - lo);
+      }
+    };
+    if (k_out) {
+      RH_CHECK(rh_kv_gather(kc_.p + off, vc_.p + off, kv_ids_dev_.p, static_cast<int>(n), bb, kv_stage_dev_.p,
+                            copy_stream_));
+      for (int i = 0; i < pieces; ++i) {
+        const std::size_t a = i * piece, len = std::min(piece, bytes - a);
+        HIP_CHECK(hipMemcpyAsync(host + a, kv_stage_dev_.p + a, len, hipMemcpyDeviceToHost, copy_stream_));
+        HIP_CHECK(hipEventRecord(kv_events_[i], copy_stream_));
+      }
+      // Every thread copies its share of every piece as the piece lands, so the copy after
+      // the last DMA is a share of one piece, not a whole piece on one thread.
+      run_shares(workers, [&](int j) {
+        for (int i = 0; i < pieces; ++i) {
+          HIP_CHECK(hipEventSynchronize(kv_events_[i]));
+          const std::size_t a = i * piece, len = std::min(piece, bytes - a);
+          user_copy(a + share_start(len, j, workers), a + share_start(len, j + 1, workers), true);
+        }
+      });
+    } else {
+      // Each share copies its pieces into the staging buffer and queues their uploads (the
+      // scatter below runs after every share's uploads are queued).
+      run_shares(workers, [&](int j) {
+        for (int i = j; i < pieces; i += workers) {
+          const std::size_t a = i * piece, len = std::min(piece, bytes - a);
+          user_copy(a, a + len, false);
+          HIP_CHECK(hipMemcpyAsync(kv_stage_dev_.p + a, host + a, len, hipMemcpyHostToDevice, copy_stream_));
+        }
+      });
+      RH_CHECK(rh_kv_scatter(kc_.p + off, vc_.p + off, kv_ids_dev_.p, static_cast<int>(n), bb, kv_stage_dev_.p,
+                             copy_stream_));
+      HIP_CHECK(hipStreamSynchronize(copy_stream_));
+    }
+    return;
+  }
+  // Small transfers: kernels gather straight into the staging buffer, and scatter out of it.
+  // Piece i: blocks [i per, ...), staged as their K, then their V.
+  const std::size_t per = std::max<std::size_t>((n + kKvPieces - 1) / kKvPieces, (kKvMinPiece + 2 * bb - 1) / (2 * bb));
+  const int pieces = static_cast<int>((n + per - 1) / per);
+  auto piece_blocks = [&](int i) { return std::min(per, n - i * per); };
+  // [a, b) of piece i's staged bytes to or from the caller's buffers.
+  auto user_copy = [&](int i, std::size_t a, std::size_t b, bool to_user) {
+    const std::size_t first = i * per, half = piece_blocks(i) * bb;
+    unsigned char* const stage = host + first * 2 * bb;
+    for (int v = 0; v < 2; ++v) {
+      const std::size_t lo = std::max(a, v * half), hi = std::min(b, (v + 1) * half);
+      if (lo >= hi) continue;
+      const std::size_t at = first * bb + lo - v * half;
+      if (to_user)
+        std::memcpy(static_cast<unsigned char*>(v ? v_out : k_out) + at, stage + lo, hi - lo);
+      else
+        std::memcpy(stage + lo, static_cast<const unsigned char*>(v ? v_in : k_in) + at, hi - lo);
     }
   };
   if (k_out) {
-    RH_CHECK(rh_kv_gather(kc_.p + off, vc_.p + off, kv_ids_dev_.p, static_cast<int>(n), bb, kv_stage_dev_.p,
-                          copy_stream_));
     for (int i = 0; i < pieces; ++i) {
-      const std::size_t a = i * piece, len = std::min(piece, bytes - a);
-      HIP_CHECK(hipMemcpyAsync(host + a, kv_stage_dev_.p + a, len, hipMemcpyDeviceToHost, copy_stream_));
+      RH_CHECK(rh_kv_gather_to_host(kc_.p + off, vc_.p + off, kv_ids_dev_.p + i * per, static_cast<int>(piece_blocks(i)), bb,
+                                    host + i * per * 2 * bb, copy_stream_));
       HIP_CHECK(hipEventRecord(kv_events_[i], copy_stream_));
     }
-    // Every thread copies its share of every piece as the piece lands, so the copy after
-    // the last DMA is a share of one piece, not a whole piece on one thread.
     run_shares(workers, [&](int j) {
       for (int i = 0; i < pieces; ++i) {
         HIP_CHECK(hipEventSynchronize(kv_events_[i]));
-        const std::size_t a = i * piece, len = std::min(piece, bytes - a);
-        const std::size_t from = share_start(len, j, workers), to = share_start(len, j + 1, workers);
-        user_copy(a + from, to - from, true);
+        const std::size_t len = 2 * piece_blocks(i) * bb;
+        user_copy(i, share_start(len, j, workers), share_start(len, j + 1, workers), true);
       }
     });
   } else {
-    // Each share copies its pieces into the staging buffer and queues their uploads (the
-    // scatter below runs after every share's uploads are queued).
     run_shares(workers, [&](int j) {
+      HIP_CHECK(hipSetDevice(device_));
       for (int i = j; i < pieces; i += workers) {
-        const std::size_t a = i * piece, len = std::min(piece, bytes - a);
-        user_copy(a, len, false);
-        HIP_CHECK(hipMemcpyAsync(kv_stage_dev_.p + a, host + a, len, hipMemcpyHostToDevice, copy_stream_));
+        user_copy(i, 0, 2 * piece_blocks(i) * bb, false);
+        RH_CHECK(rh_kv_scatter_from_host(kc_.p + off, vc_.p + off, kv_ids_dev_.p + i * per,
+                                         static_cast<int>(piece_blocks(i)), bb, host + i * per * 2 * bb, copy_stream_));
       }
     });
-    RH_CHECK(rh_kv_scatter(kc_.p + off, vc_.p + off, kv_ids_dev_.p, static_cast<int>(n), bb, kv_stage_dev_.p,
-                           copy_stream_));
     HIP_CHECK(hipStreamSynchronize(copy_stream_));
   }
 }

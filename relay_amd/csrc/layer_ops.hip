@@ -3,6 +3,7 @@
 // gather/scatter for transfers, fp32 -> fp16 conversion, int8 quantization, and the
 // reference attention kernel. Each cites the reference kernel whose contract it keeps
 // (engine/src/cuda_backend.cu). Also the C ABI's error state and device probe.
+#include <algorithm>
 #include <cmath>
 #include <string>
 
@@ -680,6 +681,35 @@ int rh_kv_gather(const void* kpool, const void* vpool, const int* blocks, int n,
                                    static_cast<hipStream_t>(stream), static_cast<uint4v*>(const_cast<void*>(kpool)),
                                    static_cast<uint4v*>(const_cast<void*>(vpool)), blocks, n, vecs,
                                    static_cast<uint4v*>(buf)));
+  return 0;
+}
+
+// The same with buf in pinned host memory, on few workgroups: PCIe is the bound, and a transfer
+// should leave the CUs to the pass that runs beside it. 4.2 MB in pieces, host copies included (us):
+// out on 8 / 16 / 64 / 128 / 2048 workgroups 111 / 99 / 90 / 93 / 94, in 141 / 109 / 92 / 93 / 98.
+constexpr unsigned kHostGrid = 64;
+
+int rh_kv_gather_to_host(const void* kpool, const void* vpool, const int* blocks, int n, size_t block_bytes, void* buf,
+                         void* stream) {
+  if (n == 0) return 0;
+  RH_REQUIRE(n > 0 && block_bytes % 16 == 0, "kv_gather_to_host: block bytes must be a multiple of 16");
+  const int64_t vecs = static_cast<int64_t>(block_bytes / 16);
+  RH_TRY_LAUNCH(hipLaunchKernelGGL(kv_pack_kernel<true>, dim3(std::min(grid_for(2 * n * vecs), kHostGrid)), dim3(kThreads), 0,
+                                   static_cast<hipStream_t>(stream), static_cast<uint4v*>(const_cast<void*>(kpool)),
+                                   static_cast<uint4v*>(const_cast<void*>(vpool)), blocks, n, vecs,
+                                   static_cast<uint4v*>(buf)));
+  return 0;
+}
+
+int rh_kv_scatter_from_host(void* kpool, void* vpool, const int* blocks, int n, size_t block_bytes, const void* buf,
+                            void* stream) {
+  if (n == 0) return 0;
+  RH_REQUIRE(n > 0 && block_bytes % 16 == 0, "kv_scatter_from_host: block bytes must be a multiple of 16");
+  const int64_t vecs = static_cast<int64_t>(block_bytes / 16);
+  RH_TRY_LAUNCH(hipLaunchKernelGGL(kv_pack_kernel<false>, dim3(std::min(grid_for(2 * n * vecs), kHostGrid)), dim3(kThreads), 0,
+                                   static_cast<hipStream_t>(stream), static_cast<uint4v*>(kpool),
+                                   static_cast<uint4v*>(vpool), blocks, n, vecs,
+                                   static_cast<uint4v*>(const_cast<void*>(buf))));
   return 0;
 }
 

@@ -318,3 +318,29 @@ def test_gather_rows(torch_mod, dev):
     assert np.array_equal(xo.cpu().numpy()[:3], x[rows]) and np.array_equal(ao.cpu().numpy()[:3], a[rows])
     assert (xo[3] == 5.0).all() and (ao[3] == 5).all()
     assert L.rh_gather_rows(X.data_ptr(), 577, A.data_ptr(), 1030, R.data_ptr(), 3, X.data_ptr(), ao.data_ptr(), None) != 0
+
+
+@pytest.mark.parametrize("n,vecs", [(1, 1), (3, 7), (40, 300)])
+def test_kv_host_transfers_equal_the_device_ones(torch_mod, dev, n, vecs):
+    """Gather into, and scatter from, pinned host memory: the bytes of rh_kv_gather / _scatter, at one
+    vector and at more vectors than one pass of the small grid covers."""
+    from relay_amd import _lib
+
+    L = _lib.lib()
+    bb, blocks = 16 * vecs, n + 5
+    rng = np.random.default_rng(n)
+    pools = [torch_mod.from_numpy(rng.integers(0, 255, blocks * bb).astype(np.uint8)).to(dev) for _ in range(2)]
+    ids = torch_mod.from_numpy(rng.permutation(blocks)[:n].astype(np.int32)).to(dev)
+    buf = torch_mod.zeros(2 * n * bb, dtype=torch_mod.uint8, device=dev)
+    host = torch_mod.zeros(2 * n * bb, dtype=torch_mod.uint8, pin_memory=True)
+    args = (pools[0].data_ptr(), pools[1].data_ptr(), ids.data_ptr(), n, bb)
+    _lib.check(L.rh_kv_gather(*args, buf.data_ptr(), None))
+    _lib.check(L.rh_kv_gather_to_host(*args, host.data_ptr(), None))
+    torch_mod.cuda.synchronize()
+    assert np.array_equal(buf.cpu().numpy(), host.numpy())
+    a, b = ([torch_mod.zeros_like(p) for p in pools] for _ in range(2))
+    _lib.check(L.rh_kv_scatter(a[0].data_ptr(), a[1].data_ptr(), ids.data_ptr(), n, bb, buf.data_ptr(), None))
+    _lib.check(L.rh_kv_scatter_from_host(b[0].data_ptr(), b[1].data_ptr(), ids.data_ptr(), n, bb, host.data_ptr(), None))
+    torch_mod.cuda.synchronize()
+    for x, y in zip(a, b):
+        assert torch_mod.equal(x, y)
