@@ -134,13 +134,18 @@ __global__ void rmsnorm_vec_kernel(const float* x, const int* rows, const float*
   }
 }
 
-// x_out[r] = x[rows[r]] (H floats), a_out[r] = a[rows[r]] (Q halves): the rows that go on past the
-// last attention. One workgroup per row; bound by its launch (3 us for 49 rows of 4096).
-__global__ void gather_rows_kernel(const float* x, int H, const half_t* a, int Q, const int* rows, float* x_out,
-                                   half_t* a_out) {
+// x_out[r] = x[rows[r]] (nx pieces of type V), a_out[r] = a[rows[r]] (na pieces): the rows that go
+// on past the last attention. Bound by its launch and one load behind the row index, so every
+// thread moves one piece: 49 rows of 4096 @GATHER@ with one workgroup per row, whose threads
+// took 32 4-byte and 2-byte pieces each.
+template <typename V>
+__global__ void gather_rows_kernel(const V* x, int nx, const V* a, int na, const int* rows, V* x_out, V* a_out) {
   const int64_t r = blockIdx.x, from = rows[r];
-  for (int i = threadIdx.x; i < H; i += kThreads) x_out[r * H + i] = x[from * H + i];
-  for (int i = threadIdx.x; i < Q; i += kThreads) a_out[r * Q + i] = a[from * Q + i];
+  const int i = blockIdx.y * kThreads + threadIdx.x;
+  if (i < nx)
+    x_out[r * nx + i] = x[from * nx + i];
+  else if (i < nx + na)
+    a_out[r * na + i - nx] = a[from * na + i - nx];
 }
 
 // ---- the K-range merge of a split product, fused into its consumer ----------------------
@@ -283,8 +288,9 @@ __global__ void qkv_post_kernel(float* qkv, const float* bias, const float* inv_
 
 // qkv_post_kernel<false> on the ksn partial planes of the qkv product (merged4, then the same
 // arithmetic per element); a thread takes four consecutive pairs, D a multiple of 8. Bound by
-// latency and the planes' reads: 512 tokens of TinyLlama (2 planes, 10.5 MB) 4.9 us, where the
-// one-plane kernel's scalar loads take 4.3 us on half the bytes.
+// latency and the planes' reads: in whole steps 5.8-7.4 us at 512 tokens of TinyLlama (3 planes, 15.7 MB),
+// 8.3-8.6 at 512 of Llama-3; the one-plane kernel, whose product writes its sums once more, 4.3 at
+// the first.
 __global__ void qkv_post_merge_kernel(const float* __restrict__ ws, int ksn, const float* __restrict__ scale, int T,
                                       const float* bias, const float* inv_freq, const int* pos, const int* seq,
                                       const int* table_off, const int* tables, half_t* kc, half_t* vc, half_t* q_out,
@@ -552,8 +558,18 @@ int rh_gather_rows(const float* x, int H, const void* a, int Q, const int* rows,
   if (R == 0) return 0;
   RH_REQUIRE(R > 0 && H > 0 && Q > 0, "gather_rows: bad shape");
   RH_REQUIRE(x && a && rows && x_out && a_out && x != x_out && a != a_out, "gather_rows: bad pointer");
-  RH_TRY_LAUNCH(hipLaunchKernelGGL(gather_rows_kernel, dim3(R), dim3(kThreads), 0, static_cast<hipStream_t>(stream), x, H,
-                                   static_cast<const half_t*>(a), Q, rows, x_out, static_cast<half_t*>(a_out)));
+  const auto launch = [&](auto piece) {
+    using V = decltype(piece);
+    const int nx = H * static_cast<int>(sizeof(float)) / static_cast<int>(sizeof(V));
+    const int na = Q * static_cast<int>(sizeof(half_t)) / static_cast<int>(sizeof(V));
+    hipLaunchKernelGGL((gather_rows_kernel<V>), dim3(R, (nx + na + kThreads - 1) / kThreads), dim3(kThreads), 0,
+                       static_cast<hipStream_t>(stream), reinterpret_cast<const V*>(x), nx,
+                       static_cast<const V*>(a), na, rows, reinterpret_cast<V*>(x_out), static_cast<V*>(a_out));
+  };
+  const bool vec = H % 4 == 0 && Q % 8 == 0 &&
+                   (reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(x_out) |
+                    reinterpret_cast<uintptr_t>(a_out)) % 16 == 0;
+  RH_TRY_LAUNCH(vec ? launch(float4{}) : launch(uint16_t{}));
   return 0;
 }
 

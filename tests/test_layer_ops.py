@@ -303,21 +303,23 @@ def test_qkv_post_to_cache_matches_qkv_post(torch_mod, dev, bs):
     assert "q_out is required" in _lib.last_error()
 
 
-def test_gather_rows(torch_mod, dev):
-    """Rows in any order, widths that are no multiple of the workgroup; the rest stays."""
+@pytest.mark.parametrize("H,Q", [(577, 1030), (576, 1032), (1020, 8), (4096, 4096)])
+def test_gather_rows(torch_mod, dev, H, Q):
+    """Rows in any order, widths that are no multiple of the workgroup, of 16 bytes or of neither; the
+    rest stays."""
     from relay_amd import _lib
 
     L = _lib.lib()
     rng = np.random.default_rng(11)
-    x, a = rng.standard_normal((9, 577)).astype(np.float32), rng.integers(0, 1 << 15, (9, 1030)).astype(np.int16)
+    x, a = rng.standard_normal((9, H)).astype(np.float32), rng.integers(0, 1 << 15, (9, Q)).astype(np.int16)
     rows = np.array([8, 0, 3], np.int32)
     X, A, R = (torch_mod.from_numpy(v).to(dev) for v in (x, a, rows))
-    xo, ao = torch_mod.full((4, 577), 5.0, device=dev), torch_mod.full((4, 1030), 5, dtype=torch_mod.int16, device=dev)
-    _lib.check(L.rh_gather_rows(X.data_ptr(), 577, A.data_ptr(), 1030, R.data_ptr(), 3, xo.data_ptr(), ao.data_ptr(), None))
+    xo, ao = torch_mod.full((4, H), 5.0, device=dev), torch_mod.full((4, Q), 5, dtype=torch_mod.int16, device=dev)
+    _lib.check(L.rh_gather_rows(X.data_ptr(), H, A.data_ptr(), Q, R.data_ptr(), 3, xo.data_ptr(), ao.data_ptr(), None))
     torch_mod.cuda.synchronize()
     assert np.array_equal(xo.cpu().numpy()[:3], x[rows]) and np.array_equal(ao.cpu().numpy()[:3], a[rows])
     assert (xo[3] == 5.0).all() and (ao[3] == 5).all()
-    assert L.rh_gather_rows(X.data_ptr(), 577, A.data_ptr(), 1030, R.data_ptr(), 3, X.data_ptr(), ao.data_ptr(), None) != 0
+    assert L.rh_gather_rows(X.data_ptr(), H, A.data_ptr(), Q, R.data_ptr(), 3, X.data_ptr(), ao.data_ptr(), None) != 0
 
 
 @pytest.mark.parametrize("n,vecs", [(1, 1), (3, 7), (40, 300)])
