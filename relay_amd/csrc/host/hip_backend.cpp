@@ -250,7 +250,7 @@ class HipBackend final : public Backend {
   // Whether an fp16 product runs the tile kernel (rh_gemm_f16) for this shape.
   static bool tiled(int K, int N, int T);
   void gemm_f16(const std::uint16_t* W, const std::uint16_t* x, float* y, int T, int K, int N, float beta);
-  // Whether gemm_f16 runs the skinny product (else the library GEMM) for this shape.
+  // Whether gemm_f16 runs the skinny product (else the tile kernel or the library) for this shape.
   static bool skinny(int K, int N, int T);
   void kv_io(int layer, const std::vector<int>& blocks, void* k_out, void* v_out, const void* k_in, const void* v_in);
   // Pieces of a large KV transfer: writes in 16, reads in 8 (each DMA piece costs ~10 us beyond
@@ -416,11 +416,11 @@ void HipBackend::load_weights(const WeightSource& src) {
 }
 
 void HipBackend::gemm_f16(const std::uint16_t* W, const std::uint16_t* x, float* y, int T, int K, int N, float beta) {
-  // Decode batch sizes up to 16 tokens: the skinny MFMA product; above, the library's timed
-  // choice. Measured on whole decode steps (ms per step, skinny / library for every plain
-  // product): TinyLlama 1.38 / 1.42 at 8 tokens, 1.51 / 1.45 at 16, 1.88 / 1.67 at 24,
-  // 2.06 / 1.70 at 32; SmolLM2-135M 1.16 / 1.28 at 8, 1.60 / 1.70 at 16, 1.66 / 1.50 at 32;
-  // one token: config 1's step 0.85 against 1.75 ms.
+  // Decode batch sizes up to 16 tokens: the skinny MFMA product; above, the tile kernel, and the
+  // library's timed choice for the largest. Skinny against library on whole decode steps (ms per
+  // step, for every plain product): TinyLlama 1.38 / 1.42 at 8 tokens, 1.51 / 1.45 at 16, 1.88 /
+  // 1.67 at 24, 2.06 / 1.70 at 32; SmolLM2-135M 1.16 / 1.28 at 8, 1.60 / 1.70 at 16, 1.66 / 1.50
+  // at 32; one token: config 1's step 0.85 against 1.75 ms.
   if (skinny(K, N, T)) {
     const int ks = rh_gemv_f16_split_plan(T, K, N);
     if (ks > 1) {
