@@ -473,6 +473,12 @@ extern "C" int rh_decode_slice_keys(int n_dec, int kv_heads, int group, int head
   // context (enough workgroups to spread over the 256 CUs), more while there are fewer
   // than 256 groups, but never below 8 chunks (one per wave of an 8-wave workgroup).
   const long groups = static_cast<long>(n_dec) * kv_heads * ((group + 15) / 16);
+  // Head size 64, short contexts: one slice; merging several costs more than a wave's second
+  // chunk. Measured (us, slices by the rules below / one): 300 keys, 9/3 heads, 1 to 16 contexts
+  // 5.9-6.7 / 5.4-6.1, 32/4 7.1-7.8 / 5.8-6.2; 448 keys 6.0-8.2 / 6.1-7.0; 512 keys, 9/3, one context 6.2 /
+  // 6.5. From 64 groups to 640 keys: 64 to 120 groups 9.2-9.9 / 7.7-8.0, 48 groups, 9/3 7.5 / 7.7.
+  if (head_dim == 64 && groups <= 128 && max_ctx <= (groups < 64 ? 7 : 10) * chunk)
+    return (max_ctx + chunk - 1) / chunk * chunk;
   // Head size 64 or 128 with few groups: the step is latency-bound, so kMergeBatch slices
   // per context (the merge then takes one round of loads), of 2 to 8 chunks, as long as that
   // makes at most 256 workgroups (longer contexts take the rule below: enough workgroups
@@ -480,8 +486,12 @@ extern "C" int rh_decode_slice_keys(int n_dec, int kv_heads, int group, int head
   // Measured (us, against the earlier 4-chunk minimum on 4 waves): 1 x 640 keys, 9/3 heads
   // (config 1) 6.87 -> 6.16; 1 x 2048, 32/4 8.57 -> 8.12; 8 x 2048, 32/4 10.78 -> 10.19;
   // 1 x 2048, 32/8, D128 11.65 -> 10.41.
+  // From 32 groups at head size 64 a slice has at least 4 chunks (2 / 4: 8 x 1024, 32/4 9.0 / 8.4,
+  // 8 x 640 8.2 / 7.8; and where 2 made too many workgroups, two slices / these: 12 x 1024 9.6 / 8.8,
+  // 16 x 1024, 9/3 9.1 / 8.3; at 24 groups, 9/3, 640 keys 2 / 4: 7.0 / 7.3).
   if (head_dim == 64 || head_dim == 128) {
-    const long small = std::max(2L * chunk, static_cast<long>((max_ctx + kMergeBatch * chunk - 1) / (kMergeBatch * chunk) * chunk));
+    const long least = (head_dim == 64 && groups >= 32 ? 4L : 2L) * chunk;
+    const long small = std::max(least, static_cast<long>((max_ctx + kMergeBatch * chunk - 1) / (kMergeBatch * chunk) * chunk));
     if (small <= 8L * chunk && groups * ((max_ctx + small - 1) / small) <= 256) return static_cast<int>(small);
   }
   // A handful of short contexts: one slice (no merge); the launch is latency-bound anyway.

@@ -240,3 +240,14 @@ def test_slices_of_several_rounds(torch_mod, dev, D, slice_keys, bs, n):
     g, counters = run_decode(torch_mod, dev, case, slice_keys=slice_keys)
     check_close(g, oracle_out(case))
     assert not counters.any()
+
+
+@pytest.mark.parametrize("heads,kv_heads,n,ctx", [(9, 3, 1, 448), (9, 3, 1, 449), (9, 3, 21, 65), (32, 4, 16, 640),
+                                                  (32, 4, 16, 641), (32, 4, 8, 1024), (32, 4, 7, 449)])
+def test_planned_slices_of_short_contexts(torch_mod, dev, heads, kv_heads, n, ctx):
+    """The planner's slices beside its lines at head size 64 (one slice, at least two or four chunks),
+    with shorter contexts in the batch."""
+    case = PagedCase([ctx] + [1 + (ctx - 1) * i // n for i in range(n - 1)], 1, heads, kv_heads, 64, 16, seed=n)
+    g, counters = run_decode(torch_mod, dev, case)
+    check_close(g, oracle_out(case))
+    assert not counters.any()
