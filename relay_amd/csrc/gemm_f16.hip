@@ -310,20 +310,24 @@ int launch_f16(int tile, const half_t* w, int64_t ldw, const half_t* x, float* y
 
 using namespace relay_hip;
 
+// Byte offsets into W (rows ldw elements apart) and x stay below 2^31.
+static bool gemm_f16_offsets_fit(int T, int K, int N, int64_t ldw) {
+  return ldw < (int64_t(1) << 30) && N * ldw < (int64_t(1) << 30) && static_cast<int64_t>(T) * K < (int64_t(1) << 30);
+}
+
 static int gemm_f16_checks(const void* w16, int64_t ldw, const void* x, int T, int K, int N) {
   RH_REQUIRE(T > 0 && N > 0 && K > 0 && K % 64 == 0, "gemm_f16: K must be a positive multiple of 64");
   RH_REQUIRE(ldw >= K && ldw % 8 == 0, "gemm_f16: ldw must be >= K and a multiple of 8");
   RH_REQUIRE(w16 != nullptr && x != nullptr, "gemm_f16: missing pointer");
   RH_REQUIRE((reinterpret_cast<uintptr_t>(w16) | reinterpret_cast<uintptr_t>(x)) % 16 == 0,
              "gemm_f16: W16 and x must be 16-byte aligned");
-  RH_REQUIRE(static_cast<int64_t>(T) * K < (int64_t(1) << 30) && ldw < (int64_t(1) << 30) / N,
+  RH_REQUIRE(gemm_f16_offsets_fit(T, K, N, ldw),
              "gemm_f16: T * K or N * ldw too large for 32-bit buffer offsets");
   return 0;
 }
 
 extern "C" int rh_gemm_f16_fits(int T, int K, int N) {
-  return T > 0 && N > 0 && K > 0 && K % 64 == 0 && static_cast<int64_t>(T) * K < (int64_t(1) << 30) &&
-         static_cast<int64_t>(N) * K < (int64_t(1) << 30) - K;
+  return T > 0 && N > 0 && K > 0 && K % 64 == 0 && gemm_f16_offsets_fit(T, K, N, K);
 }
 
 extern "C" int rh_gemm_f16(const void* w16, int64_t ldw, const void* x, float* y, int T, int K, int N, float beta,

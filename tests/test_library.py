@@ -53,6 +53,21 @@ def test_no_device_means_an_error_not_a_fallback():
         HipBackend(w, 8, 16)
 
 
+@pytest.mark.parametrize("T,K,N", [(32, 4096, 262080), (32, 4096, 262081), (32, 4096, 262100), (32, 4096, 262142),
+                                   (32, 4096, 262143), (32, 4096, 262144), (17, 8192, 131070), (17, 8192, 131071),
+                                   (17, 8192, 131072), (262143, 4096, 64), (262144, 4096, 64), (20, 64, 16777215),
+                                   (20, 64, 16777216), (33, 576, 1864135), (33, 576, 1864136)])
+def test_gemm_f16_takes_every_shape_that_fits_says(T, K, N):
+    """rh_gemm_f16_fits says whether rh_gemm_f16 takes a shape with ldw = K, on both sides of N * K and
+    T * K = 2^30. y is misaligned, so that the call ends in a refusal whatever the shape."""
+    lib = _lib.lib()
+    assert lib.rh_gemm_f16(16, K, 16, 4, T, K, N, 0.0, None) != 0
+    refused = "too large" in _lib.last_error()
+    assert refused or "y must be 16-byte aligned" in _lib.last_error()
+    assert lib.rh_gemm_f16_fits(T, K, N) == (0 if refused else 1)
+    assert refused == (max(T, N) * K >= 1 << 30)
+
+
 def test_kernel_launchers_validate_shapes_before_launching():
     lib = _lib.lib()
     assert lib.rh_gemv_int8(None, 64, None, 0, None, None, 0, 64, 64, 0.0, None) != 0
