@@ -534,6 +534,10 @@ int relay_hip_backend_read_kv_block(relay_hip_backend* b, int layer, int block, 
 int relay_hip_backend_write_kv_block(relay_hip_backend* b, int layer, int block, const void* k_in, const void* v_in);
 int relay_hip_backend_read_kv_layer(relay_hip_backend* b, int layer, const int* blocks, int n, void* out);
 int relay_hip_backend_write_kv_layer(relay_hip_backend* b, int layer, const int* blocks, int n, const void* in);
+/* Blocks until the layer's K/V writes of the pass that is running are done, from any thread; at
+ * once when none runs. The first wait that finds a pass running returns when that pass is over:
+ * passes record an event per layer only from then on (with relay's C++ interface also from the
+ * first pass with an observer), and later waits return with their layer. */
 int relay_hip_backend_wait_kv_written(relay_hip_backend* b, int layer);
 
 /* Backend::update_weight (backend.h:74-80): `name` as relay names weights, src fp32 in

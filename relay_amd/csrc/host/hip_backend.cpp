@@ -11,7 +11,7 @@
 //    reference issues seven); the prefill work (rh_prefill_plan) pairs light and heavy
 //    causal row blocks and comes heaviest first, so the imbalance does not leave CUs
 //    idle at the end of the kernel;
-//  - one event per layer after its KV write backs wait_kv_written in observed passes, and KV block traffic
+//  - one event per layer after its KV write backs wait_kv_written (on backends that use it), and KV block traffic
 //    runs on a second stream under its own mutex (cuda_backend.cu:611-664).
 // Errors are C++ exceptions as in the reference: std::invalid_argument for bad batches,
 // std::out_of_range for token ids, std::runtime_error("HIP: ...") for runtime failures.
@@ -21,7 +21,6 @@
 #include <algorithm>
 #include <atomic>
 #include <cmath>
-#include <condition_variable>
 #include <cstdlib>
 #include <cstring>
 #include <exception>
@@ -52,6 +51,7 @@ HipOptions HipOptions::from_env() {
 namespace {
 
 using relay_hip_host::DeviceArray;
+using relay_hip_host::KvProgress;
 using relay_hip_host::PinnedBuffer;
 using relay_hip_host::LtGemm;
 
@@ -91,7 +91,7 @@ class HipBackend final : public Backend {
  public:
   HipBackend(const ModelConfig& c, const WeightSource& src, int num_blocks, int block_size, int device,
              int max_tokens, int max_context, HipOptions options)
-      : c_(c), opt_(options), max_tokens_(max_tokens), max_context_(max_context), device_(device) {
+      : c_(c), opt_(options), max_tokens_(max_tokens), max_context_(max_context), device_(device), progress_(c.layers) {
     if (num_blocks <= 0 || block_size <= 0) throw std::invalid_argument("num_blocks and block_size must be positive");
     if (max_tokens <= 0) throw std::invalid_argument("max_batch_tokens must be positive");
     if (c.heads <= 0 || c.kv_heads <= 0 || c.heads % c.kv_heads) throw std::invalid_argument("bad head counts");
@@ -174,12 +174,7 @@ class HipBackend final : public Backend {
   }
   void wait_kv_written(int layer) override {
     const hipEvent_t done = layer_done_.at(layer);
-    {
-      // A pass without an observer records no event per layer: its layers are written when it
-      // is over.
-      std::unique_lock<std::mutex> lock(pass_mu_);
-      pass_over_.wait(lock, [&] { return !unobserved_pass_; });
-    }
+    progress_.reach(layer);
     HIP_CHECK(hipEventSynchronize(done));
   }
 
@@ -213,27 +208,6 @@ class HipBackend final : public Backend {
   static constexpr int kLogitThreads = 3;
   static constexpr std::size_t kLogitThreadBytes = std::size_t(2) << 20;
   std::vector<hipEvent_t> logit_events_;
-  // Set while a pass without an observer runs. Only an observed pass records layer_done_ events
-  // (relay's sender waits for a layer once the observer has named it): an event between two
-  // kernels costs 3 us on the device and 4 us of the launching thread (SmolLM2-135M, one token,
-  // 30 layers: 910 -> 777 us a step, 756 -> 668 on the device).
-  struct UnobservedPass {
-    HipBackend& b;
-    bool on;
-    UnobservedPass(HipBackend& be, bool unobserved) : b(be), on(unobserved) { set(true); }
-    ~UnobservedPass() { set(false); }
-    void set(bool running) {
-      if (!on) return;
-      {
-        std::lock_guard<std::mutex> lock(b.pass_mu_);
-        b.unobserved_pass_ = running;
-      }
-      if (!running) b.pass_over_.notify_all();
-    }
-  };
-  std::mutex pass_mu_;
-  std::condition_variable pass_over_;
-  bool unobserved_pass_ = false;
   bool pending_ = false;  // a pass was enqueued and not yet finished
   void load_weights(const WeightSource& src);
   DeviceMatrix make_matrix(const float* host, int N, int K, const WeightSource& src, std::uint64_t stream_id);
@@ -275,6 +249,7 @@ class HipBackend final : public Backend {
   rocblas_handle blas_ = nullptr;
   std::unique_ptr<LtGemm> lt_;  // timed-choice hipBLASLt products (rocBLAS if it has none)
   std::vector<hipEvent_t> layer_done_;
+  KvProgress progress_;
   hipEvent_t fwd_begin_ = nullptr, fwd_end_ = nullptr;
   double last_ms_ = 0;
 
@@ -550,7 +525,7 @@ void HipBackend::gemm(const DeviceMatrix& W, const std::uint16_t* x, float* y, i
 }
 
 std::vector<float> HipBackend::forward(const ForwardBatch& batch, LayerObserver* observer) {
-  UnobservedPass pass(*this, !observer);
+  KvProgress::Pass pass(progress_, observer != nullptr);
   const std::size_t n = enqueue_forward(batch, observer, std::numeric_limits<std::size_t>::max());
   std::vector<float> out(n);
   finish_forward(out.data(), n);
@@ -558,7 +533,7 @@ std::vector<float> HipBackend::forward(const ForwardBatch& batch, LayerObserver*
 }
 
 int HipBackend::forward_into(const ForwardBatch& batch, float* dst, std::size_t cap) {
-  UnobservedPass pass(*this, true);
+  KvProgress::Pass pass(progress_, false);
   const std::size_t n = enqueue_forward(batch, nullptr, cap);
   finish_forward(dst, n);
   return static_cast<int>(n / c_.vocab);
@@ -741,10 +716,11 @@ std::size_t HipBackend::enqueue_forward(const ForwardBatch& batch, LayerObserver
                              c_.heads, c_.kv_heads, D, layout_.block_size, stream_));
     }
     attn_xn_ready = false;
-    if (observer) {
+    if (progress_.record()) {
       HIP_CHECK(hipEventRecord(layer_done_[l], stream_));
-      observer->kv_written(l);
+      progress_.recorded(l);
     }
+    if (observer) observer->kv_written(l);
     if (fast_attention_) {
       if (n_work)
         RH_CHECK(rh_flash_prefill(qh_.p, Q, kc, vc, d_tab, d_work, n_work, c_.heads, c_.kv_heads, D,

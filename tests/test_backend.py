@@ -302,3 +302,40 @@ def test_rows_without_logits_are_dropped_after_the_last_attention(dev, int8):
             assert np.array_equal(a.read_kv_layer(layer, list(range(40))), b.read_kv_layer(layer, list(range(40))))
     step = lambda be: be.forward(ForwardBatch([SeqChunk([7], len(p), t, True) for p, t in zip(prompts, tab)]))
     assert np.array_equal(step(a), step(b))
+
+
+def test_wait_kv_written_beside_passes(dev):
+    """A thread that waits for layers and reads them while another runs passes back to back: every
+    wait ends, and a read after the last pass has that pass's bytes."""
+    import threading
+
+    w = small_model(64, 8, 2, layers=3, hidden=512, inter=768)
+    be, alone = HipBackend(w, 40, 16, options=FAST), HipBackend(w, 40, 16, options=FAST)
+    tokens = np.random.default_rng(9).integers(0, 512, 300).tolist()
+    batch = ForwardBatch([SeqChunk(tokens, 0, list(range(40)), True)])
+    stop, done, failed = threading.Event(), [0], []
+
+    def wait():
+        try:
+            while done[0] < 60:
+                be.wait_kv_written(done[0] % 3)
+                be.read_kv_layer(done[0] % 3, list(range(40)))
+                done[0] += 1
+        except Exception as e:  # noqa: BLE001 (the assertion below shows it)
+            failed.append(e)
+        stop.set()
+
+    be.forward(batch)
+    t = threading.Thread(target=wait, daemon=True)
+    t.start()
+    passes = 0
+    while not stop.is_set() and passes < 5000:
+        be.forward(batch)
+        passes += 1
+    t.join(timeout=30)
+    assert not failed and done[0] == 60, (failed, done[0], passes)
+    want = alone.forward(batch)
+    assert np.array_equal(be.forward(batch), want)
+    for layer in range(3):
+        be.wait_kv_written(layer)
+        assert np.array_equal(be.read_kv_layer(layer, list(range(40))), alone.read_kv_layer(layer, list(range(40))))
