@@ -389,6 +389,12 @@ int rh_f16_merge_rmsnorm(const float* workspace, int ksplit, int T, int H, float
 int rh_gemm_f16_gate_up_silu(const void* w16, int64_t ldw, const void* x, void* act, int T, int K, int I, void* stream);
 int rh_gemm_f16_gate_up_plan(int T, int K, int I);
 
+/* 1 where the tile kernel is measured at least level with the library product, by what happens to
+ * its outputs: stored whole (rh_gemm_f16), left as K ranges to a consumer that adds them
+ * (rh_gemm_f16_partials), or through SiLU * mul (N = 2 I). 0 also for shapes it cannot take. */
+enum { RH_F16_PLAIN = 0, RH_F16_RANGES = 1, RH_F16_SILU = 2 };
+int rh_gemm_f16_pays(int T, int K, int N, int form);
+
 /* Per-row symmetric int8 quantization of an fp32 matrix [N, K] on the device:
  * scale[n] = max_k |w[n, k]| / 127 (1 if the row is all zero), q = round-half-even(w / scale),
  * q rows ldq bytes apart (ldq >= K; the bytes past K are not written).

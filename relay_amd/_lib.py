@@ -91,6 +91,7 @@ SIGNATURES = {
     "rh_f16_merge_rmsnorm": (I, [P, I, I, I, P, P, F, P, P]),
     "rh_gemm_f16_gate_up_silu": (I, [P, I64, P, P, I, I, I, P]),
     "rh_gemm_f16_gate_up_plan": (I, [I, I, I]),
+    "rh_gemm_f16_pays": (I, [I, I, I, I]),
     "rh_gemv_f16_rmsnorm": (I, [P, I64, P, P, F, P, I, I, I, F, P]),
     "rh_gemv_f16_silu": (I, [P, I64, P, P, I, I, I, F, P]),
     "rh_gemv_f16_fused_fits": (I, [I, I]),

@@ -330,6 +330,28 @@ extern "C" int rh_gemm_f16_fits(int T, int K, int N) {
   return T > 0 && N > 0 && K > 0 && K % 64 == 0 && gemm_f16_offsets_fit(T, K, N, K);
 }
 
+// Where the tile kernel is at least level with hipBLASLt's fastest kernel for the same shape
+// (timed on that token count, with the launches that each side needs for its consumer: qkv_post,
+// the RMSNorm after o and down, SiLU * mul; us, library / tile). Weights N x K, T tokens:
+// - Products whose ranges the consumer adds, below 4 M outputs: 4096 x 4096 at 512 35 / 34, 4096 x
+//   14336 at 512 78 / 75, 6144 x 4096 at 560 52 / 49, 2048 x 5632 at 1024 43 / 41; 2048 x 2048 at 768
+//   19 / 22 and at 32 9 / 10 (level in whole passes). Past them the library fills the chip with
+//   larger tiles: 6144 x 4096 at 1536 84 / 114, 4096 x 14336 186 / 212, 2048 x 5632 at 3072 80 / 93.
+// - Plain products only where the plan would not split either; one that has to walk all of K on
+//   few workgroups is far behind: 5120 x 13824 at 32 39 / 76, 8192 x 8192 at 64 44 / 62. (LM heads of fewer
+//   outputs stay here although the library is ahead, 32000 x 2048 at 32 25 / 31, 128256 x 4096 at 17 161 /
+//   182: under 1% of a pass, and its choice by timing adds 17-75 ms to a program's first one.)
+// - SiLU in the epilogue, below 10 M outputs, and with K <= 2048 always: 11264 x 2048 at 512 41 / 32,
+//   at 2048 115 / 105, 28672 x 4096 at 256 83 / 76, at 384 100 / 125.
+//   Not with 100 M weights and more at up to 64 tokens: that is a stream of weights, which the
+//   library reads at 6 TB/s and this kernel at 5: 28672 x 4096 at 32 44 / 47, 27648 x 5120 at 64 57 / 64.
+extern "C" int rh_gemm_f16_pays(int T, int K, int N, int form) {
+  if (!rh_gemm_f16_fits(T, K, N)) return 0;
+  const int64_t weights = static_cast<int64_t>(N) * K, outputs = static_cast<int64_t>(T) * N;
+  if (form == RH_F16_SILU) return (outputs < 10000000 || K <= 2048) && (T > 64 || weights < 100000000);
+  return outputs < 4000000 && (form == RH_F16_RANGES || f16_plan(T, K, N, 0).ks == 1);
+}
+
 extern "C" int rh_gemm_f16(const void* w16, int64_t ldw, const void* x, float* y, int T, int K, int N, float beta,
                            void* stream) {
   if (T == 0) return 0;

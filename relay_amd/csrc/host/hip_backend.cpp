@@ -221,8 +221,8 @@ class HipBackend final : public Backend {
   float* w8_split_ws(int ks, int T, int N);
   int w8_partials(const DeviceMatrix& W, const std::uint16_t* x, int T);
   int partials(const DeviceMatrix& W, const std::uint16_t* x, int T);
-  // Whether an fp16 product runs the tile kernel (rh_gemm_f16) for this shape.
-  static bool tiled(int K, int N, int T);
+  // Whether an fp16 product runs the tile kernel for this shape; form: an RH_F16_* of rh_gemm_f16_pays.
+  static bool tiled(int K, int N, int T, int form);
   void gemm_f16(const std::uint16_t* W, const std::uint16_t* x, float* y, int T, int K, int N, float beta);
   // Whether gemm_f16 runs the skinny product (else the tile kernel or the library) for this shape.
   static bool skinny(int K, int N, int T);
@@ -410,7 +410,7 @@ void HipBackend::gemm_f16(const std::uint16_t* W, const std::uint16_t* x, float*
     RH_CHECK(rh_gemv_f16_splitk(W, K, x, y, T, K, N, beta, ks, split_ws_.p, split_counters_.p, stream_));
     return;
   }
-  if (tiled(K, N, T) && W != dequant_.p) {
+  if (W != dequant_.p && tiled(K, N, T, RH_F16_PLAIN)) {
     RH_CHECK(rh_gemm_f16(W, K, x, y, T, K, N, beta, stream_));
     return;
   }
@@ -433,14 +433,7 @@ bool HipBackend::skinny(int K, int N, int T) {
   return K % 16 == 0 && (T <= 16 || (T <= 32 && static_cast<std::int64_t>(N) * K < (std::int64_t{1} << 22)));
 }
 
-bool HipBackend::tiled(int K, int N, int T) {
-  // The library's 256 x 256 kernels stay ahead on the largest products: library / tile kernel
-  // in isolation (us) 53 / 72 at 384 x 32000 outputs (K = 2048), 91 / 113 at 2048 x 6144
-  // (4096), 108 / 130 at 512 x 28672 (4096); 35 / 34 at 512 x 11264 (2048), 68 / 73 at 2048 x
-  // 4096 (4096), 93 / 72 at 512 x 4096 (14336), 58 / 53 at 2048 x 2048 (5632), 32 / 9.6 at
-  // 256 x 2048 (2048).
-  return !skinny(K, N, T) && rh_gemm_f16_fits(T, K, N) && static_cast<std::int64_t>(T) * N < 10000000;
-}
+bool HipBackend::tiled(int K, int N, int T, int form) { return !skinny(K, N, T) && rh_gemm_f16_pays(T, K, N, form); }
 
 bool HipBackend::fused(const DeviceMatrix& W, int T, bool int8_ok) const {
   // Normalisation / activation folded into the skinny fp16 product, up to 16 tokens, when its
@@ -479,7 +472,7 @@ int HipBackend::w8_partials(const DeviceMatrix& W, const std::uint16_t* x, int T
 // plan (rh_f16_merge_* and rh_qkv_post_merge add them).
 int HipBackend::partials(const DeviceMatrix& W, const std::uint16_t* x, int T) {
   if (W.i8.p) return w8_partials(W, x, T);
-  if (!tiled(W.K, W.N, T) || W.N % 4) return 0;
+  if (!tiled(W.K, W.N, T, RH_F16_RANGES) || W.N % 4) return 0;
   const int ks = rh_gemm_f16_partials_plan(T, W.K, W.N);
   if (ks < 2) return 0;
   RH_CHECK(rh_gemm_f16_partials(W.f16.p, W.K, x, T, W.K, W.N, ks, w8_split_ws(ks, T, W.N), stream_));
@@ -780,12 +773,9 @@ std::size_t HipBackend::enqueue_forward(const ForwardBatch& batch, LayerObserver
         const bool tile_silu = L.w_gate_up.i8.p && Tl > 64 && rh_gemm_w8_plan(Tl, H, 2 * I) == 1 &&
                                rh_gemm_w8_kernel(Tl, H, 2 * I, 1) == 1 &&
                                (static_cast<std::int64_t>(I) + 256) * L.w_gate_up.ldw < (std::int64_t(1) << 31);
-        // fp16 above the whole-line kernel's range: SiLU·mul in the tile kernel's epilogue. On
-        // products large enough for the library that saves the fp32 [T, 2 I] round trip and
-        // a launch, which outweighs the library's faster kernel while K is short (2048 tokens
-        // of TinyLlama: 104 us against 97 + 22; 512 of Llama-3-8B: 130 against 106 + 12).
-        const bool f16_tile = !L.w_gate_up.i8.p && !skinny(H, 2 * I, Tl) &&
-                              (tiled(H, 2 * I, Tl) || (H <= 2048 && rh_gemm_f16_fits(Tl, H, 2 * I)));
+        // fp16 above the whole-line kernel's range: SiLU·mul in the tile kernel's epilogue, which
+        // saves the fp32 [T, 2 I] round trip and a launch.
+        const bool f16_tile = !L.w_gate_up.i8.p && tiled(H, 2 * I, Tl, RH_F16_SILU);
         const int ks = tile_silu || f16_tile || I % 8 ? 0 : w8_partials(L.w_gate_up, xn_.p, Tl);
         if (f16_tile) {
           const int gks = rh_gemm_f16_gate_up_plan(Tl, H, I);

@@ -68,6 +68,29 @@ def test_gemm_f16_takes_every_shape_that_fits_says(T, K, N):
     assert refused == (max(T, N) * K >= 1 << 30)
 
 
+PLAIN, RANGES, SILU = 0, 1, 2  # RH_F16_*
+
+
+@pytest.mark.parametrize("T,K,N,form,pays", [
+    # A plain product that the plan would split has no one to add its ranges: o and down of widths
+    # past the merging RMSNorm's 4096 (library / tile us: 39 / 76, 44 / 62, 37 / 76).
+    (32, 13824, 5120, PLAIN, 0), (64, 8192, 8192, PLAIN, 0), (17, 13824, 5120, PLAIN, 0), (32, 5632, 2048, PLAIN, 0),
+    (32, 5632, 2048, RANGES, 1), (560, 576, 960, PLAIN, 1), (560, 4096, 6144, RANGES, 1),
+    # 4 M outputs (1536 x 6144: 84 / 114; 3072 x 2048, K 5632: 80 / 93).
+    (1536, 4096, 6144, RANGES, 0), (1536, 14336, 4096, RANGES, 0), (3072, 5632, 2048, RANGES, 0), (3999, 1024, 1000, RANGES, 1),
+    (4000, 1024, 1000, RANGES, 0),
+    # SiLU in the epilogue: 10 M outputs where K is past 2048.
+    (512, 2048, 11264, SILU, 1), (2048, 2048, 11264, SILU, 1), (256, 4096, 28672, SILU, 1), (384, 4096, 28672, SILU, 0),
+    # The same with 100 M weights and more at up to 64 tokens (44 / 47, 57 / 64).
+    (32, 4096, 28672, SILU, 0), (64, 5120, 27648, SILU, 0), (65, 4096, 28672, SILU, 1), (64, 2048, 11264, SILU, 1),
+    # LM heads, for their first pass's sake.
+    (32, 2048, 32000, PLAIN, 1), (17, 4096, 128256, PLAIN, 1), (32, 4096, 128256, PLAIN, 0),
+    # Shapes that the kernel cannot take.
+    (32, 96, 64, RANGES, 0), (20, 64, 1 << 24, PLAIN, 0)])
+def test_f16_tile_kernel_is_chosen_where_it_is_level_or_ahead(T, K, N, form, pays):
+    assert _lib.lib().rh_gemm_f16_pays(T, K, N, form) == pays
+
+
 def test_kernel_launchers_validate_shapes_before_launching():
     lib = _lib.lib()
     assert lib.rh_gemv_int8(None, 64, None, 0, None, None, 0, 64, 64, 0.0, None) != 0
