@@ -455,7 +455,7 @@ int rh_kv_scatter(void* kpool, void* vpool, const int* blocks, int n, size_t blo
                   void* stream);
 
 /* The same with buf in pinned host memory that the device can address, on few workgroups (PCIe
- * is the bound, and a transfer should leave the CUs to the pass that runs beside it). */
+ * is the bound). They hold their CUs for the whole transfer: for times when no pass runs. */
 int rh_kv_gather_to_host(const void* kpool, const void* vpool, const int* blocks, int n, size_t block_bytes, void* buf,
                          void* stream);
 int rh_kv_scatter_from_host(void* kpool, void* vpool, const int* blocks, int n, size_t block_bytes, const void* buf,

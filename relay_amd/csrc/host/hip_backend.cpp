@@ -230,14 +230,19 @@ class HipBackend final : public Backend {
   // Pieces of a large KV transfer: writes in 16, reads in 8 (each DMA piece costs ~10 us beyond
   // its bytes, and a read's host copies are split over the threads; Llama-3 layer reads of 33.6
   // MB: 34.1 GB/s at 16 pieces, 36.9-38.8 at 8, 38.5-39.1 at 4, 28-31 at 2; writes 35.5 at 16,
-  // 34-36 at 8, 30.5 at 4). Up to 8 MB kernels read and write the pinned staging buffer
-  // themselves, in up to 16 pieces of at least 512 KB: no device copy and no DMA set-up per piece
-  // (4.2 MB: write 125 -> 92 us, read 112 -> 92; 0.5 MB: 50 -> 34, 55 -> 38; at 33.6 MB level within
-  // the runs' spread, writes 870 by DMA, 960-1020 by kernels).
+  // 34-36 at 8, 30.5 at 4). Up to 8 MB, and while no pass runs, kernels read and write the
+  // pinned staging buffer themselves, in up to 16 pieces of at least 512 KB: no device copy and no
+  // DMA set-up per piece (4.2 MB: write 125 -> 92 us, read 112 -> 92; 0.5 MB: 50 -> 34, 55 -> 38; at 33.6
+  // MB level within the runs' spread, writes 870 by DMA, 960-1020 by kernels). Beside a pass the DMA
+  // engine moves them: the kernels' waves sit on CUs for the whole PCIe time, and products that
+  // take a CU's registers whole wait for them (device time of a pass beside back-to-back
+  // transfers of 4.2 MB, alone / by DMA / by kernels: two Llama-3 layers, 16 sequences 337 / 358 / 450,
+  // 48 and a 464-token chunk 705 / 723 / 870-1020; four TinyLlama layers, 512-token chunk 418 / 444 /
+  // 580-620).
   static constexpr int kKvPieces = 16, kKvReadPieces = 8;
   static constexpr std::size_t kKvDirect = std::size_t(8) << 20;
   static constexpr int kKvThreads = 4;  // host threads copying them (8: no faster)
-  static constexpr std::size_t kKvMinPiece = std::size_t(512) << 10;
+  static constexpr std::size_t kKvMinPiece = std::size_t(512) << 10, kKvMinDma = std::size_t(1) << 20;
   std::vector<hipEvent_t> kv_events_;                           // one per piece in flight
 
   ModelConfig c_;
@@ -945,14 +950,14 @@ void HipBackend::kv_io(int layer, const std::vector<int>& blocks, void* k_out, v
   }
   // The host-side copies between the caller's buffers and the pinned staging run on a few
   // threads (one core moves ~10-25 GB/s; the transfers run at the PCIe rate).
-  const int workers = bytes >= kLogitThreadBytes ? kKvThreads : 1;
-  if (bytes > kKvDirect) {
+  const int threads = bytes >= kLogitThreadBytes ? kKvThreads : 1;
+  if (bytes > kKvDirect || progress_.running()) {
     // Staging bytes [0, n bb) are K, [n bb, 2 n bb) V, here and on the device; the DMA engine
     // moves them in pieces, piece i [i piece, (i + 1) piece).
     if (kv_stage_dev_.n < bytes) kv_stage_dev_ = DeviceArray<unsigned char>(bytes);
     const int chunks = k_out ? kKvReadPieces : kKvPieces;
-    const std::size_t piece = (bytes + chunks - 1) / chunks;
-    const int pieces = static_cast<int>((bytes + piece - 1) / piece);
+    const std::size_t piece = std::max(kKvMinDma, (bytes + chunks - 1) / chunks);
+    const int pieces = static_cast<int>((bytes + piece - 1) / piece), workers = std::min(threads, pieces);
     auto user_copy = [&](std::size_t from, std::size_t to, bool to_user) {
       for (int v = 0; v < 2; ++v) {
         const std::size_t lo = std::max(from, v * n * bb), hi = std::min(to, (v + 1) * n * bb);
@@ -999,7 +1004,7 @@ void HipBackend::kv_io(int layer, const std::vector<int>& blocks, void* k_out, v
   // Small transfers: kernels gather straight into the staging buffer, and scatter out of it.
   // Piece i: blocks [i per, ...), staged as their K, then their V.
   const std::size_t per = std::max<std::size_t>((n + kKvPieces - 1) / kKvPieces, (kKvMinPiece + 2 * bb - 1) / (2 * bb));
-  const int pieces = static_cast<int>((n + per - 1) / per);
+  const int pieces = static_cast<int>((n + per - 1) / per), workers = std::min(threads, pieces);
   auto piece_blocks = [&](int i) { return std::min(per, n - i * per); };
   // [a, b) of piece i's staged bytes to or from the caller's buffers.
   auto user_copy = [&](int i, std::size_t a, std::size_t b, bool to_user) {

@@ -700,9 +700,10 @@ int rh_kv_gather(const void* kpool, const void* vpool, const int* blocks, int n,
   return 0;
 }
 
-// The same with buf in pinned host memory, on few workgroups: PCIe is the bound, and a transfer
-// should leave the CUs to the pass that runs beside it. 4.2 MB in pieces, host copies included (us):
-// out on 8 / 16 / 64 / 128 / 2048 workgroups 111 / 99 / 90 / 93 / 94, in 141 / 109 / 92 / 93 / 98.
+// The same with buf in pinned host memory, on few workgroups, since PCIe is the bound. For a device
+// with nothing else to do: the workgroups stay on their CUs for the whole PCIe time, which makes
+// a forward pass beside them 30-60% slower. 4.2 MB in pieces, host copies included (us): out on 8 / 16 /
+// 64 / 128 / 2048 workgroups 111 / 99 / 90 / 93 / 94, in 141 / 109 / 92 / 93 / 98.
 constexpr unsigned kHostGrid = 64;
 
 int rh_kv_gather_to_host(const void* kpool, const void* vpool, const int* blocks, int n, size_t block_bytes, void* buf,

@@ -339,3 +339,58 @@ def test_wait_kv_written_beside_passes(dev):
     for layer in range(3):
         be.wait_kv_written(layer)
         assert np.array_equal(be.read_kv_layer(layer, list(range(40))), alone.read_kv_layer(layer, list(range(40))))
+
+
+@pytest.mark.parametrize("beside", [False, True])
+@pytest.mark.parametrize("kv_heads,bs", [(2, 16), (3, 5)])
+def test_kv_transfers_of_several_pieces(dev, kv_heads, bs, beside):
+    """KV blocks written and read together against the same blocks one at a time, on both sides of
+    every line in a transfer's size: pieces (512 KB, short last ones; 1 MB by DMA), threads (2 MB),
+    kernels to DMA (8 MB), with block sizes whose K/V border lies inside a thread's share; alone,
+    and beside passes that run back to back on other blocks, where the DMA engine moves them all."""
+    import threading
+
+    w = small_model(64, 2 * kv_heads, kv_heads, hidden=128, inter=128)
+    bb = kv_heads * bs * 64 * 2
+    at = lambda mb: int(mb * (1 << 20)) // (2 * bb)
+    sizes = sorted({at(0.5) - 1, at(0.5) + 1, at(1) + 1, at(2) - 1, at(2) + 1, at(2.6), at(8) - 1, at(8) + 1, at(9.1)})
+    own, nb = 40, 40 + at(9.1) + 8  # blocks 0 .. 39 belong to the passes
+    be = HipBackend(w, nb, bs, max_batch_tokens=256, options=FAST)
+    assert be.kv_block_bytes() == bb
+    rng = np.random.default_rng(bs)
+    prompt = rng.integers(0, 512, 200).tolist()
+    batch = ForwardBatch([SeqChunk(prompt, 0, list(range(own)), True)])
+    want = be.forward(batch)
+    stop, failed = threading.Event(), []
+
+    def passes():
+        while not stop.is_set():
+            if not np.array_equal(be.forward(batch), want):
+                failed.append(1)
+
+    thread = threading.Thread(target=passes, daemon=True)
+    if beside:
+        thread.start()
+    try:
+        for n in sizes:
+            print(f"kv transfer case: {n} blocks of {bb} bytes, beside={beside}", flush=True)
+            blocks = (own + rng.permutation(nb - own)[:n + 1]).tolist()
+            kept = blocks.pop()
+            before = be.read_kv_block(1, kept)
+            data = rng.integers(0, 256, 2 * n * bb, dtype=np.uint8)
+            be.write_kv_layer(1, blocks, data)
+            k, v = data[:n * bb].reshape(n, bb), data[n * bb:].reshape(n, bb)
+            for i in {*range(0, n, 37), *range(max(0, n - 3), n), *range(min(n, 66))}:
+                got = be.read_kv_block(1, blocks[i])
+                assert np.array_equal(got[0], k[i]) and np.array_equal(got[1], v[i]), (n, i)
+            for a, b in zip(before, be.read_kv_block(1, kept)):
+                assert np.array_equal(a, b)
+            order = rng.permutation(n)
+            back = be.read_kv_layer(1, [blocks[i] for i in order])
+            assert np.array_equal(back, np.concatenate([k[order].ravel(), v[order].ravel()])), n
+    finally:
+        stop.set()
+        if beside:
+            thread.join(timeout=30)
+    assert not failed and np.array_equal(be.forward(batch), want)
+    be.close()
