@@ -203,8 +203,10 @@ class HipBackend final : public Backend {
   // Each D2H piece costs ~10 us of its own beyond its bytes, each helper thread ~15 us to start.
   // Whole steps with 4.1 / 6.3 MB of logits (us): 256 KB pieces on 3 threads 646 / 1065, 512 KB 533 /
   // 1007, 1 MB 475 / 929, 2 MB 456 / 907, 4 MB 490 / 915; 2 MB on 1, 2, 4, 6 threads 506, 459, 458, 497 /
-  // 974, 912, 909, 944.
-  static constexpr std::size_t kLogitMinPiece = std::size_t(2) << 20;
+  // 974, 912, 909, 944. Up to 2 MB, on one thread, in pieces of 1 MB, so that the first is copied
+  // under the second's DMA (beyond the pass, 32,000-token logits of 12 / 16 rows: 115 / 130 us, in one
+  // piece 126 / 157).
+  static constexpr std::size_t kLogitSmallPiece = std::size_t(1) << 20, kLogitPiece = std::size_t(2) << 20;
   static constexpr int kLogitThreads = 3;
   static constexpr std::size_t kLogitThreadBytes = std::size_t(2) << 20;
   std::vector<hipEvent_t> logit_events_;
@@ -894,7 +896,7 @@ void HipBackend::finish_forward(float* dst, std::size_t n) {
       logit_events_.resize(kLogitChunks);
       for (auto& e : logit_events_) HIP_CHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     }
-    piece = std::max(kLogitMinPiece, (bytes + kLogitChunks - 1) / kLogitChunks);
+    piece = std::max(bytes >= kLogitThreadBytes ? kLogitPiece : kLogitSmallPiece, (bytes + kLogitChunks - 1) / kLogitChunks);
     piece = (piece + 255) & ~std::size_t(255);
     pieces = static_cast<int>((bytes + piece - 1) / piece);
     auto* host = static_cast<unsigned char*>(logits_host_.p);

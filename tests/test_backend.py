@@ -394,3 +394,18 @@ def test_kv_transfers_of_several_pieces(dev, kv_heads, bs, beside):
             thread.join(timeout=30)
     assert not failed and np.array_equal(be.forward(batch), want)
     be.close()
+
+
+def test_logits_of_several_pieces(dev):
+    """Every row of the logits reaches the caller, on both sides of the pieces' lines (1 MB pieces up
+    to 2 MB of logits, then 2 MB ones shared by three threads)."""
+    w = small_model(64, 2, 1, layers=1, vocab=32768, hidden=64, inter=64)  # 128 KB a row
+    rng = np.random.default_rng(3)
+    rows = 49
+    chunks = [SeqChunk([int(t)], 0, [i], True) for i, t in enumerate(rng.integers(0, 32768, rows))]
+    want = O.CpuBackend(w, rows, 16).forward(ForwardBatch(chunks))
+    be = HipBackend(w, rows, 16, options=FAST)
+    for n in (1, 7, 8, 9, 15, 16, 17, 31, 32, 33, 49):
+        got = be.forward(ForwardBatch(chunks[:n]))
+        assert got.shape == (n, 32768) and rel_err_rowmax(got, want[:n]) < 1e-2, n
+    be.close()
