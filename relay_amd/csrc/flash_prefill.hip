@@ -180,22 +180,23 @@ __global__ __launch_bounds__(kThreads) void flash_prefill_kernel(const PrefillAr
     const int qpos = p0 + row;
     const int wave_last = p0 + min(strip * 32 + 31, nrows - 1);  // last key any row of the strip sees
 
-    auto lookup = [&](int k0) {
+    // (end: keys of the tile that are wanted.)
+    auto lookup = [&](int k0, int end) {
 #pragma unroll
       for (int i = 0; i < LOADS; ++i) {
         int kl, cc;
-        if (item(i, kl, cc)) {
+        if (item(i, kl, cc) && (end == kKeyTile || kl < end)) {
           // Keys past the block's last are masked for every row; read a valid row instead.
           const int key = min(k0 + kl, nkeys - 1);
           blk[i] = table[POW2 ? key >> sh : key / bs];
         }
       }
     };
-    auto fetch = [&](int k0) {
+    auto fetch = [&](int k0, int end) {
 #pragma unroll
       for (int i = 0; i < LOADS; ++i) {
         int kl, cc;
-        if (item(i, kl, cc)) {
+        if (item(i, kl, cc) && (end == kKeyTile || kl < end)) {
           const int key = min(k0 + kl, nkeys - 1);
           const int slot = POW2 ? key & (bs - 1) : key % bs;
           const int64_t off = kv_row_offset(blk[i], a.kv_heads, kvh, bs, slot, DR) + 8 * cc;
@@ -209,11 +210,11 @@ __global__ __launch_bounds__(kThreads) void flash_prefill_kernel(const PrefillAr
         }
       }
     };
-    auto store = [&](int buf) {
+    auto store = [&](int buf, int end) {
 #pragma unroll
       for (int i = 0; i < LOADS; ++i) {
         int kl, cc;
-        if (item(i, kl, cc)) {
+        if (item(i, kl, cc) && (end == kKeyTile || kl < end)) {
           const int off = kl * D + ((cc ^ kswz<D>(kl)) << 3);
           *reinterpret_cast<half8*>(sK + buf * KBUF + off) = kreg[i];
           // V row-major like K (the PV operands come out of LDS through transposing reads).
@@ -361,19 +362,86 @@ __global__ __launch_bounds__(kThreads) void flash_prefill_kernel(const PrefillAr
     // tile j, barrier; the loads are in flight under the compute.
     const int ntiles = (nkeys + kKeyTile - 1) / kKeyTile;
     __syncthreads();  // the previous phase's merge is done with the LDS
-    lookup(0);
-    fetch(0);
-    if (ntiles > 1) lookup(kKeyTile);
-    store(0);
-    if (ntiles > 1) fetch(kKeyTile);
-    if (ntiles > 2) lookup(2 * kKeyTile);
+    if constexpr (SPLIT > 2 && D <= 64) {
+      // A context of one tile: only the parts that hold a key are staged and merged, in code of its
+      // own so that the loop below keeps its schedule (us, prompts of 8 / 64 / 100 tokens, all parts /
+      // these: 9 heads 6.4 / 4.5, 6.5 / 5.2, 6.5 / 5.7; in 128-row workgroups 5.1, 5.5, 6.2).
+      if (ntiles == 1) {
+        const int end = (nkeys + 32 * kSub - 1) / (32 * kSub) * (32 * kSub);
+        lookup(0, end);
+        fetch(0, end);
+        store(0, end);
+        __syncthreads();
+        if (wave_on && 32 * kSub * half <= wave_last) compute(std::true_type{}, 0, 32 * kSub * half);
+        __syncthreads();
+        const int parts = wave_last / (32 * kSub) + 1;  // of this strip
+        float* const xs = reinterpret_cast<float*>(smem) + strip * (SPLIT - 1) * XSTRIP;
+        if (half && half < parts) {
+          float* const xo = xs + (half - 1) * XSTRIP;
+#pragma unroll
+          for (int i = 0; i < DT; ++i)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) xo[(i * 16 + r) * 64 + lane] = o[i][r];
+          xo[DT * 16 * 64 + lane] = ref;
+          xo[DT * 16 * 64 + 64 + lane] = l_part;
+        }
+        if (end > 32 * kSub) __syncthreads();
+        if (!half && row_ok) {
+          float f[SPLIT], m = ref;
+#pragma unroll
+          for (int p = 1; p < SPLIT; ++p)
+            if (p < parts) m = fmaxf(m, xs[(p - 1) * XSTRIP + DT * 16 * 64 + lane]);
+          f[0] = fast_exp2(ref - m);
+          float l = l_part * f[0];
+#pragma unroll
+          for (int p = 1; p < SPLIT; ++p)
+            if (p < parts) {
+              const float* const xml = xs + (p - 1) * XSTRIP + DT * 16 * 64;
+              f[p] = xml[lane] == -INFINITY ? 0.0f : fast_exp2(xml[lane] - m);
+              l += xml[64 + lane] * f[p];
+            }
+          const float inv = 1.0f / (l + xlane_sum(l));
+          half_t* orow = a.out + static_cast<int64_t>(t0 + row) * a.out_stride + static_cast<int64_t>(head) * DR;
+#pragma unroll
+          for (int dt = 0; dt < DT; ++dt) {
+            float ov[16];
+#pragma unroll
+            for (int r = 0; r < 16; ++r) ov[r] = o[dt][r] * f[0];
+#pragma unroll
+            for (int p = 1; p < SPLIT; ++p)
+              if (p < parts) {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) ov[r] += xs[(p - 1) * XSTRIP + (dt * 16 + r) * 64 + lane] * f[p];
+              }
+#pragma unroll
+            for (int r4 = 0; r4 < 4; ++r4) {
+              half4 v;
+#pragma unroll
+              for (int j = 0; j < 4; ++j) v[j] = static_cast<half_t>(ov[4 * r4 + j] * inv);
+              if (DR == D || 32 * dt + 8 * r4 + 4 * hh < DR)
+                *reinterpret_cast<half4*>(orow + 32 * dt + 8 * r4 + 4 * hh) = v;
+            }
+          }
+        }
+        continue;
+      }
+    }
+    // (Head size 128: the registers leave no room for that path; the first tile is staged up to its
+    // last part with a key, and the merge below has a form for one or two parts.)
+    const int end0 = SPLIT > 2 && D == 128 && ntiles == 1 ? (nkeys + 31) / 32 * 32 : kKeyTile;
+    lookup(0, end0);
+    fetch(0, end0);
+    if (ntiles > 1) lookup(kKeyTile, kKeyTile);
+    store(0, end0);
+    if (ntiles > 1) fetch(kKeyTile, kKeyTile);
+    if (ntiles > 2) lookup(2 * kKeyTile, kKeyTile);
     __syncthreads();
     const int first_masked = p0 + strip * 32 - 32 * kSub * (half + 1) + 1;  // unmasked: j * kKeyTile <= this
     const int j_mask = min(ntiles, first_masked >= 0 ? first_masked / kKeyTile + 1 : 0);
     auto prepare = [&](int j) {
-      if (j + 1 < ntiles) store((j + 1) & 1);
-      if (j + 2 < ntiles) fetch((j + 2) * kKeyTile);
-      if (j + 3 < ntiles) lookup((j + 3) * kKeyTile);
+      if (j + 1 < ntiles) store((j + 1) & 1, kKeyTile);
+      if (j + 2 < ntiles) fetch((j + 2) * kKeyTile, kKeyTile);
+      if (j + 3 < ntiles) lookup((j + 3) * kKeyTile, kKeyTile);
     };
     int j = 0;
     for (; j < j_mask; ++j) {
@@ -388,6 +456,40 @@ __global__ __launch_bounds__(kThreads) void flash_prefill_kernel(const PrefillAr
       __syncthreads();
     }
 
+    if constexpr (SPLIT > 2 && D == 128) {
+      // At most two parts with a key (us, 8 / 64 tokens, 32 heads, all parts / these: 7.4 / 6.2, 8.0 / 7.0;
+      // 512 rows at position 7680 101.6 / 103.0).
+      if (nkeys <= 64) {
+        float* const xo = reinterpret_cast<float*>(smem) + strip * XSTRIP;
+        if (half == 1) {
+#pragma unroll
+          for (int i = 0; i < DT; ++i)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) xo[(i * 16 + r) * 64 + lane] = o[i][r];
+          xo[DT * 16 * 64 + lane] = ref;
+          xo[DT * 16 * 64 + 64 + lane] = l_part;
+        }
+        __syncthreads();
+        if (!half && row_ok) {
+          const float mp = xo[DT * 16 * 64 + lane], m = fmaxf(ref, mp);
+          const float f0 = fast_exp2(ref - m), f1 = mp == -INFINITY ? 0.0f : fast_exp2(mp - m);
+          const float l = l_part * f0 + xo[DT * 16 * 64 + 64 + lane] * f1;
+          const float inv = 1.0f / (l + xlane_sum(l));
+          half_t* orow = a.out + static_cast<int64_t>(t0 + row) * a.out_stride + static_cast<int64_t>(head) * DR;
+#pragma unroll
+          for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+            for (int r4 = 0; r4 < 4; ++r4) {
+              half4 v;
+#pragma unroll
+              for (int j = 0; j < 4; ++j)
+                v[j] = static_cast<half_t>((o[dt][4 * r4 + j] * f0 + xo[(dt * 16 + 4 * r4 + j) * 64 + lane] * f1) * inv);
+              *reinterpret_cast<half4*>(orow + 32 * dt + 8 * r4 + 4 * hh) = v;
+            }
+        }
+        continue;
+      }
+    }
     // Merge the strip's parts: the others' (max, sum, O^T) through LDS (the tile buffers are
     // free after the loop's last barrier) into the first part's wave, which saw key 0, so its
     // offset is finite; the others' may not be.

@@ -138,6 +138,19 @@ def test_row_cuts(torch_mod, dev, heads, kv_heads, D, bs, rows, start):
     check_close(run_prefill(torch_mod, dev, case), oracle_out(case))
 
 
+@pytest.mark.parametrize("rows", [3, 300])
+@pytest.mark.parametrize("keys", [1, 31, 32, 33, 63, 64, 65, 96, 97, 127, 128, 129, 160, 255, 256, 257])
+@pytest.mark.parametrize("heads,kv_heads,D,bs", [(8, 2, 64, 16), (96, 4, 64, 12), (12, 3, 32, 16), (6, 2, 16, 16),
+                                                 (16, 4, 128, 16), (16, 2, 128, 5)])
+def test_contexts_of_one_tile(torch_mod, dev, heads, kv_heads, D, bs, keys, rows):
+    """Contexts of at most one tile of a cut launch, where only the parts that hold a key are staged
+    and merged, and the next ones: on both sides of every part's first key (32 keys a part, 4 or 8
+    parts), for the last rows of a context and for whole prompts, with another chunk beside."""
+    rows = min(rows, keys)
+    case = PagedCase([keys, 40], [rows, 2], heads, kv_heads, D, bs, seed=keys + rows)
+    check_close(run_prefill(torch_mod, dev, case), oracle_out(case))
+
+
 def test_gather_is_bit_exact_under_permutation(torch_mod, dev):
     case = PagedCase([400], [400], 8, 2, 64, 16, seed=1)
     a = run_prefill(torch_mod, dev, case)
