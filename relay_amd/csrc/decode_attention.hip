@@ -486,30 +486,35 @@ extern "C" int rh_decode_slice_keys(int n_dec, int kv_heads, int group, int head
   // Measured (us, against the earlier 4-chunk minimum on 4 waves): 1 x 640 keys, 9/3 heads
   // (config 1) 6.87 -> 6.16; 1 x 2048, 32/4 8.57 -> 8.12; 8 x 2048, 32/4 10.78 -> 10.19;
   // 1 x 2048, 32/8, D128 11.65 -> 10.41.
-  // From 32 groups at head size 64 a slice has at least 4 chunks (2 / 4: 8 x 1024, 32/4 9.0 / 8.4,
-  // 8 x 640 8.2 / 7.8; and where 2 made too many workgroups, two slices / these: 12 x 1024 9.6 / 8.8,
-  // 16 x 1024, 9/3 9.1 / 8.3; at 24 groups, 9/3, 640 keys 2 / 4: 7.0 / 7.3).
+  // From 32 groups at head size 64 a slice has at least 4 chunks where that still makes three (2 /
+  // 4: 8 x 1024, 32/4 9.0 / 8.4, 8 x 640 8.2 / 7.8; and where 2 made too many workgroups, two slices / these:
+  // 12 x 1024 9.6 / 8.8, 16 x 1024, 9/3 9.1 / 8.3; at 24 groups, 9/3, 640 keys 2 / 4: 7.0 / 7.3; two slices
+  // of 4: 12 x 460, 9/3 6.7 / 7.5, 16 x 512 7.2 / 7.7, 12 x 512, 32/4 7.9 / 8.1).
   if (head_dim == 64 || head_dim == 128) {
-    const long least = (head_dim == 64 && groups >= 32 ? 4L : 2L) * chunk;
+    const long least = (head_dim == 64 && groups >= 32 && max_ctx > 8 * chunk ? 4L : 2L) * chunk;
     const long small = std::max(least, static_cast<long>((max_ctx + kMergeBatch * chunk - 1) / (kMergeBatch * chunk) * chunk));
     if (small <= 8L * chunk && groups * ((max_ctx + small - 1) / small) <= 256) return static_cast<int>(small);
   }
   // A handful of short contexts: one slice (no merge); the launch is latency-bound anyway.
   if (groups <= 16 && max_ctx <= 16 * chunk) return (max_ctx + chunk - 1) / chunk * chunk;
-  long parts = std::max(2L, 256 / groups);
+  const auto keys_of = [&](long parts) {
+    const long per_part = (max_ctx + parts - 1) / parts;
+    return std::max(8L * chunk, (per_part + chunk - 1) / chunk * chunk);
+  };
+  long keys = keys_of(std::max(2L, 256 / groups));
   // Past one workgroup per CU with two slices: the fewest slices that fill whole rounds of 256
   // workgroups to 85% (else the fullest). Measured (us, 2 slices / these): 144 groups, 9/3 heads,
   // D64, 8192 keys 68.5 / 52 (ragged 54 / 37), 192 groups, 32/4, D64, 4096 keys 42.5 / 38.1 (ragged 31.2 /
-  // 23.9); 384 groups fill three rounds with two.
+  // 23.9); 384 groups fill three rounds with two. Slices that the 8-chunk minimum makes fewer and
+  // fuller of gaps are counted as they are: 192 groups, 32/4, 1500 keys 18.1 in two, 20.1 in three.
   if (groups > 128) {
     double best = 0.0;
     for (long p = 2; p <= kMergeBatch && best < 0.85; ++p) {
-      const double fill = static_cast<double>(groups * p) / ((groups * p + 255) / 256 * 256);
-      if (fill > best) best = fill, parts = p;
+      const long k = keys_of(p), wgs = groups * ((max_ctx + k - 1) / k);
+      const double fill = static_cast<double>(wgs) / ((wgs + 255) / 256 * 256);
+      if (fill > best) best = fill, keys = k;
     }
   }
-  const long per_part = (max_ctx + parts - 1) / parts;
-  const long keys = std::max(8L * chunk, (per_part + chunk - 1) / chunk * chunk);
   return static_cast<int>(keys);
 }
 

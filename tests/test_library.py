@@ -68,6 +68,17 @@ def test_gemm_f16_takes_every_shape_that_fits_says(T, K, N):
     assert refused == (max(T, N) * K >= 1 << 30)
 
 
+@pytest.mark.parametrize("n,kv_heads,group,D,ctx,keys", [
+    # 32 to 63 (context, kv head) groups of head size 64: slices of 4 chunks only where that makes three.
+    (12, 3, 3, 64, 460, 128), (16, 3, 3, 64, 512, 128), (12, 4, 8, 64, 512, 128), (16, 3, 3, 64, 513, 256), (8, 4, 8, 64, 640, 256),
+    # Past 128 groups rounds are filled by the slices that there are, at least 8 chunks each: a third
+    # slice fills no more of them (192 groups), or does (144).
+    (48, 4, 8, 64, 1500, 768), (64, 3, 3, 64, 1500, 768), (24, 8, 4, 128, 700, 352), (48, 3, 3, 64, 1500, 512),
+    (48, 4, 8, 64, 4096, 1024), (48, 4, 8, 64, 2048, 512)])
+def test_decode_slices(n, kv_heads, group, D, ctx, keys):
+    assert _lib.lib().rh_decode_slice_keys(n, kv_heads, group, D, ctx) == keys
+
+
 PLAIN, RANGES, SILU = 0, 1, 2  # RH_F16_*
 
 
