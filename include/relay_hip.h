@@ -377,6 +377,8 @@ int rh_gemm_f16_fits(int T, int K, int N);
 int rh_gemm_f16_partials(const void* w16, int64_t ldw, const void* x, int T, int K, int N, int ksplit,
                          float* workspace, void* stream);
 int rh_gemm_f16_partials_plan(int T, int K, int N);
+/* The output tile that either form runs for this shape and split: 1000 * rows of W + tokens. */
+int rh_gemm_f16_tile(int T, int K, int N, int ksplit);
 int rh_f16_merge_silu(const float* workspace, int ksplit, int T, int I, void* act, void* stream);
 int rh_f16_merge_rmsnorm(const float* workspace, int ksplit, int T, int H, float* x, const float* norm_w, float eps,
                          void* out, void* stream);

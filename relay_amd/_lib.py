@@ -92,6 +92,7 @@ SIGNATURES = {
     "rh_gemm_f16_gate_up_silu": (I, [P, I64, P, P, I, I, I, P]),
     "rh_gemm_f16_gate_up_plan": (I, [I, I, I]),
     "rh_gemm_f16_pays": (I, [I, I, I, I]),
+    "rh_gemm_f16_tile": (I, [I, I, I, I]),
     "rh_gemv_f16_rmsnorm": (I, [P, I64, P, P, F, P, I, I, I, F, P]),
     "rh_gemv_f16_silu": (I, [P, I64, P, P, I, I, I, F, P]),
     "rh_gemv_f16_fused_fits": (I, [I, I]),

@@ -45,8 +45,8 @@ __global__ __launch_bounds__(WN * WT * WK * 64, 1) void gemm_f16_kernel(const ha
   constexpr int KS = 64, WAVES = WN * WT * WK, Q = 4 / WK, AN = BN / WN / 32, AT = BT / WT / 32;
   constexpr int ROWS = BN + BT, PIECES = ROWS / 8;  // a piece: 8 rows x 128 bytes, one wave load
   constexpr int LPS = (PIECES + WAVES - 1) / WAVES;             // loads per wave and stage
-  constexpr bool SPREAD = STAGES > 2;                // the next stage's loads spread over the step
-  constexpr int AHEAD = SPREAD ? STAGES - 1 : STAGES; // stages issued before the first step
+  constexpr int AHEAD = STAGES - 1;                  // stages issued before the first step
+  static_assert(STAGES >= 3, "a stage's loads are spread over the step two stages before its own");
   static_assert(WK == 1 || STAGES * ROWS * 128 >= BN * BT * 4, "the K halves meet in the ring");
   static_assert(BN % (32 * WN) == 0 && BT % (32 * WT) == 0, "tile");
   constexpr int STAGE = ROWS * KS;                  // halves per stage: W rows, then x rows
@@ -142,7 +142,7 @@ __global__ __launch_bounds__(WN * WT * WK * 64, 1) void gemm_f16_kernel(const ha
 #pragma unroll
     for (int q = 0; q + 1 < Q; ++q) {
       read(buf, q + 1, (q + 1) & 1);
-      if (SPREAD && more) issue(s + STAGES - 1, pbuf, q, Q - 1);
+      if (more) issue(s + STAGES - 1, pbuf, q, Q - 1);
       mma(q & 1);
     }
     if (s + 1 < nsteps) {
@@ -152,7 +152,6 @@ __global__ __launch_bounds__(WN * WT * WK * 64, 1) void gemm_f16_kernel(const ha
       asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");
       wait_stages<LPS, STAGES - 2>(nsteps - 2 - s);
       ring_barrier();
-      if (!SPREAD && s + STAGES < nsteps) issue(s + STAGES, buf, 0, 1);
       read(nbuf, 0, 0);
     }
     mma((Q - 1) & 1);
@@ -360,6 +359,12 @@ extern "C" int rh_gemm_f16(const void* w16, int64_t ldw, const void* x, float* y
   return launch_f16<kStore>(f16_plan(T, K, N, 1).tile, static_cast<const half_t*>(w16), ldw,
                             static_cast<const half_t*>(x), y, T, K, N, beta, 1, nullptr,
                             static_cast<hipStream_t>(stream));
+}
+
+extern "C" int rh_gemm_f16_tile(int T, int K, int N, int ksplit) {
+  if (T < 1 || K <= 0 || K % 64 || N <= 0 || ksplit < 1 || ksplit > kMaxF16Split) return -1;
+  const F16Tile& t = kTiles[f16_plan(T, K, N, ksplit).tile];
+  return t.rows * 1000 + t.toks;
 }
 
 extern "C" int rh_gemm_f16_partials_plan(int T, int K, int N) {

@@ -136,7 +136,7 @@ __global__ void rmsnorm_vec_kernel(const float* x, const int* rows, const float*
 
 // x_out[r] = x[rows[r]] (nx pieces of type V), a_out[r] = a[rows[r]] (na pieces): the rows that go
 // on past the last attention. Bound by its launch and one load behind the row index, so every
-// thread moves one piece: 49 rows of 4096 @GATHER@ with one workgroup per row, whose threads
+// thread moves one piece: 49 rows of 4096 5.0 us, 11.0 with one workgroup per row, whose threads
 // took 32 4-byte and 2-byte pieces each.
 template <typename V>
 __global__ void gather_rows_kernel(const V* x, int nx, const V* a, int na, const int* rows, V* x_out, V* a_out) {

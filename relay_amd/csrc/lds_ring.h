@@ -1,5 +1,5 @@
 // Global memory -> LDS loads without registers, and the waits of a ring of LDS buffers fed by
-// them (the tile products of gemm_f16.hip and gemm_w8.hip).
+// them (the tile product of gemm_f16.hip).
 #pragma once
 
 #include "common.h"

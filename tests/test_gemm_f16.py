@@ -10,8 +10,8 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 EPS32 = 2.0 ** -24
-# Edges of every tile (64 x 64 to 256 x 128 rows x tokens, chosen by the plan): one token and
-# one quad of rows, a token or row past a tile, N not a multiple of 4, one 64-k step to many.
+# One token and one quad of rows, a token or row past a tile, N not a multiple of 4, one 64-k step
+# to many, on the three smallest tiles; the edges of all six are below (test_every_tile).
 SHAPES = [(1, 4, 64), (17, 100, 128), (64, 64, 576), (65, 129, 192), (129, 1000, 1536), (200, 577, 320),
           (300, 2500, 256), (513, 3000, 448), (520, 6146, 128)]
 
@@ -105,6 +105,80 @@ def test_gate_up_silu(torch_mod, dev, T, I, K):
         _lib.check(L.rh_f16_merge_silu(ws.data_ptr(), 2, T, I, act.data_ptr(), None), "merge_silu")
         torch_mod.cuda.synchronize()
         assert (np.abs(act.cpu().numpy().astype(np.float64) - want) <= bound).all()
+
+
+# (rows of W, tokens) of the tiles and the stages of their LDS rings.
+STAGES = {(64, 64): 4, (128, 64): 3, (128, 128): 4, (192, 128): 3, (256, 128): 3, (128, 256): 3}
+
+
+def shape_on(L, rows, toks, steps, form):
+    """The smallest T and N whose product of `steps` 64-k steps (a range of two for "ranges") runs this
+    tile with one token past a tile and the fewest rows past one."""
+    ks = 2 if form == "ranges" else 1
+    past = {"plain": 1, "silu": 2, "ranges": 4}[form]
+    best = None
+    for a in range(40):
+        for b in range(24):
+            T, N = a * toks + 1, b * rows + past
+            if (best is None or T * N < best[0] * best[1]) and L.rh_gemm_f16_tile(T, 64 * steps * ks, N, ks) == 1000 * rows + toks:
+                best = (T, N)
+    return best
+
+
+@pytest.mark.parametrize("form", ["plain", "silu", "ranges"])
+@pytest.mark.parametrize("rows,toks,steps", [(r, t, n) for (r, t), s in STAGES.items()
+                                             for n in (1, s - 1, s, s + 1, 2 * s + 1, 3 * s + 2)
+                                             if (r, t, n) != (192, 128, 1)])  # which the plan never runs
+def test_every_tile(torch_mod, dev, rows, toks, steps, form):
+    """Every tile and form at its row and token tails, with a ring that is not filled, just filled and
+    refilled to its last buffer and past it; nothing is written past the outputs."""
+    from relay_amd import _lib
+
+    L, torch = _lib.lib(), torch_mod
+    shape = shape_on(L, rows, toks, steps, form)
+    assert shape is not None
+    T, N = shape
+    ks = 2 if form == "ranges" else 1
+    K, ldw, beta = 64 * steps * ks, 64 * steps * ks + 8, float(steps % 2)
+    print(f"gemm_f16 tile case: {rows} x {toks} {form} T={T} N={N} K={K}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(1000 * rows + toks + steps)
+    w = (torch.randn(N, ldw, generator=g, device=dev) * 0.05).half()
+    x = torch.randn(T, K, generator=g, device=dev).half()
+    wd, xd = w[:, :K].double(), x.double()
+    tail = 4096
+
+    def product(k0, k1):
+        a, b = xd[:, k0:k1].contiguous(), wd[:, k0:k1].contiguous()
+        return a @ b.T, 4 * (k1 - k0) * EPS32 * (a.abs() @ b.abs().T) + 1e-30
+
+    if form == "plain":
+        out = torch.randn(T * N + tail, generator=g, device=dev)
+        y0 = out.clone()
+        _lib.check(L.rh_gemm_f16(w.data_ptr(), ldw, x.data_ptr(), out.data_ptr(), T, K, N, beta, None), "rh_gemm_f16")
+        want, bound = product(0, K)
+        added = beta * y0[:T * N].view(T, N).double()
+        want = want + added
+        bound = bound + 2 * EPS32 * (want.abs() + added.abs())
+        assert bool(((out[:T * N].view(T, N).double() - want).abs() <= bound).all())
+        assert torch.equal(out[T * N:], y0[T * N:])
+    elif form == "ranges":
+        out = torch.full((ks * T * N + tail,), float("nan"), device=dev)
+        _lib.check(L.rh_gemm_f16_partials(w.data_ptr(), ldw, x.data_ptr(), T, K, N, ks, out.data_ptr(), None), "partials")
+        for z in range(ks):
+            want, bound = product(64 * steps * z, 64 * steps * (z + 1))
+            assert bool(((out[z * T * N:(z + 1) * T * N].view(T, N).double() - want).abs() <= bound).all()), z
+        assert bool(out[ks * T * N:].isnan().all())
+    else:
+        I = N // 2
+        out = torch.full((T * I + tail,), float("nan"), device=dev, dtype=torch.float16)
+        _lib.check(L.rh_gemm_f16_gate_up_silu(w.data_ptr(), ldw, x.data_ptr(), out.data_ptr(), T, K, I, None), "silu")
+        y, b = product(0, K)
+        gate, u, bg, bu = y[:, :I], y[:, I:], b[:, :I], b[:, I:]
+        s = gate * torch.sigmoid(gate)
+        want = s * u  # the bound as in silu_bound
+        bound = 1.1 * bg * u.abs() + s.abs() * bu + 1.1 * bg * bu + want.abs() * (2.0 ** -11 + 16 * EPS32) + 2.0 ** -25
+        assert bool(((out[:T * I].view(T, I).double() - want).abs() <= bound).all())
+        assert bool(out[T * I:].isnan().all())
 
 
 @pytest.mark.parametrize("ks,scaled", [(1, False), (3, False), (2, True)])
