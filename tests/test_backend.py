@@ -409,3 +409,20 @@ def test_logits_of_several_pieces(dev):
         got = be.forward(ForwardBatch(chunks[:n]))
         assert got.shape == (n, 32768) and rel_err_rowmax(got, want[:n]) < 1e-2, n
     be.close()
+
+
+def test_kv_transfers_of_one_large_block(dev):
+    """A block of 2 MB read alone (by DMA), written alone and moved with another: the same bytes."""
+    w = small_model(64, 8, 8, layers=1, hidden=64, inter=64)
+    be = HipBackend(w, 4, 1024, max_batch_tokens=16, options=FAST)
+    bb = be.kv_block_bytes()
+    assert bb == 1 << 20
+    data = np.random.default_rng(6).integers(0, 256, 4 * bb, dtype=np.uint8)
+    be.write_kv_layer(0, [2, 0], data)
+    for i, block in enumerate((2, 0)):
+        k, v = be.read_kv_block(0, block)
+        assert np.array_equal(k, data[i * bb:(i + 1) * bb]) and np.array_equal(v, data[(2 + i) * bb:(3 + i) * bb])
+        be.write_kv_block(0, 3 - block, v, k)  # swapped, into blocks 1 and 3
+    back = be.read_kv_layer(0, [3, 1]).reshape(4, bb)
+    assert np.array_equal(back, data.reshape(4, bb)[[3, 2, 1, 0]])
+    be.close()
